@@ -129,6 +129,10 @@ inline int tb_plan_steps(int plan) { return plan & 0xFF; }
 // a run of 8-step launches (BGK lattices; 0 when there is none).
 int tb_remainder_plan(const cs_lattice* l, int plan);
 void launch_tb(cs_lattice* l, int plan);
+// The streaming variant of the temporally blocked step (lattice_ts.hip):
+// whether this lattice takes it, and one launch of k (8 or 4) steps.
+bool ts_takes(const cs_lattice* l);
+void launch_ts(cs_lattice* l, int k);
 // The render passes of the current populations into d_out (device, h*w pixels
 // of `channels` bytes: 3 = RGB, 4 = RGBA with alpha 255), enqueued on the
 // lattice's stream; allocates the lattice's render scratch on first use.

@@ -1520,9 +1520,14 @@ __global__ void k_check_reciprocal(unsigned long long* __restrict__ bad, float o
     unsigned int n = 0;
     for (uint32_t k = 0; k < 256u; ++k) {
         const float b = __builtin_bit_cast(float, (uint32_t)(base + k));
-        const float ref = one / b, got = recip_rn(b);
-        const bool same = __builtin_bit_cast(uint32_t, ref) == __builtin_bit_cast(uint32_t, got) ||
-                          (ref != ref && got != got);
+        Cells<float, 2> c;  // both reciprocals of the step kernels
+        c.v[0] = b;
+        c.v[1] = 1.0f;
+        const float ref = one / b, got[2] = {recip_rn(b), recip_rn(c).v[0]};
+        bool same = true;
+        for (const float g : got)
+            same = same && (__builtin_bit_cast(uint32_t, ref) == __builtin_bit_cast(uint32_t, g) ||
+                            (ref != ref && g != g));
         n += same ? 0u : 1u;
     }
     if (n) atomicAdd(bad, (unsigned long long)n);

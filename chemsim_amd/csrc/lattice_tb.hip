@@ -8,7 +8,8 @@
 // microseconds per step: one-step vector kernel 203; K = 2 197, K = 4 137,
 // K = 6 125, K = 8 116 -- beyond 8 the halo's recomputation outgrows the
 // saved traffic; with the region in registers K = 6 measured slower than 8
-// too).  Lattices of more than TB_SMALL_MAX_REGIONS 32 x 32 regions (about
+// too).  Large lattices without half-way walls take the streaming kernel
+// (lattice_ts.hip).  Otherwise lattices of more than TB_SMALL_MAX_REGIONS 32 x 32 regions (about
 // 512^2) take 64 x 64 regions: k_step_tbr (the region in registers, 73 us
 // per step at 4096^2) without geometry and in the reference boundary mode,
 // k_step_tb (the region in LDS) in the half-way mode, whose link and Zou-He
@@ -122,6 +123,7 @@ void launch_edge(cs_lattice* l, int plan)
     else launch_mode<St, CS_EDGE_ZERO>(l, plan);
 }
 
+constexpr int TS_PLAN = 1;  // in the place of a region side: the streaming kernel (lattice_ts.hip)
 constexpr int tb_plan(int k, int edge) { return k | (edge << 8); }
 
 }  // namespace
@@ -136,6 +138,7 @@ int tb_steps(const cs_lattice* l, int cpt_override)
     if ((int64_t)l->h * l->pitch * 4 >= ((int64_t)1 << 32)) return 0;  // 32-bit offsets
     if (k == CS_TEMPORAL_AUTO) {
         if (l->params.collision == CS_COLL_KBC) return 0;
+        if (ts_takes(l)) return tb_plan(8, TS_PLAN);
         constexpr int INS = TB_EDGE_SMALL - 2 * 8;
         const int64_t small = (int64_t)((l->w + INS - 1) / INS) * ((l->h + INS - 1) / INS);
         return tb_plan(8, small <= TB_SMALL_MAX_REGIONS ? TB_EDGE_SMALL : TB_EDGE);
@@ -153,6 +156,10 @@ int tb_remainder_plan(const cs_lattice* l, int plan)
 
 void launch_tb(cs_lattice* l, int plan)
 {
+    if ((plan >> 8) == TS_PLAN) {
+        launch_ts(l, tb_plan_steps(plan));
+        return;
+    }
     if (l->storage == CS_F32) launch_edge<StF32>(l, plan);
     else launch_edge<StF32Dev>(l, plan);
 }
@@ -167,3 +174,9 @@ extern "C" int cs_set_temporal_steps(int k)
         g_tb_steps.store(k, std::memory_order_relaxed);
     });
 }
+
+// The library's Makefile compiles the streaming kernel's units on their own,
+// in parallel; a build that lists only this one gets them here.
+#ifndef CS_TS_UNITS
+#include "lattice_ts.hip"
+#endif

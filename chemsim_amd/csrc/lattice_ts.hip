@@ -1,0 +1,83 @@
+// Launches of the streaming temporally blocked step kernel (lbm_ts.hpp) for
+// single lattices: which lattices take it, how the rows are split over waves,
+// and the template dispatch.
+//
+// A strip of rows costs a fill of K - 1 rows whatever its length, so the
+// streaming kernel needs a lattice that keeps every SIMD busy with long runs;
+// the region kernels (lbm_tb.hpp) recompute a fixed share instead.  Both
+// shares are known before the launch, so the choice compares them: computed
+// cells per kept cell, the streaming kernel's times 1.12 (what its instruction
+// mix costs more per computed cell; the ratio of measured times to computed
+// cells at 1536^2 .. 8192^2 is 1.07 .. 1.14).  FP32 Taylor-Green, GLUPS,
+// streaming / regions in registers: 1024^2 110 / 174, 1536^2 187 / 218,
+// 2048^2 198 / 194, 3072^2 263 / 228, 4096^2 306 / 242, 8192^2 350 / 254.
+#include "lattice_ts.hpp"
+#include "lbm_tb.hpp"
+
+using namespace cs;
+
+namespace {
+
+template <class St, int EDGE, int MODE>
+void ts_coll(cs_lattice* l, int k)
+{
+    if (k == 4) {  // the remainder launch, BGK only
+        ts_launch<St, EDGE, MODE, 4, CS_COLL_BGK>(l);
+        return;
+    }
+    if constexpr (std::is_same_v<St, StF32>) {
+        if (l->params.collision == CS_COLL_TRT) {
+            ts_launch<St, EDGE, MODE, 8, CS_COLL_TRT>(l);
+            return;
+        }
+        if (l->params.collision == CS_COLL_REGULARIZED) {
+            ts_launch<St, EDGE, MODE, 8, CS_COLL_REGULARIZED>(l);
+            return;
+        }
+    }
+    ts_launch<St, EDGE, MODE, 8, CS_COLL_BGK>(l);
+}
+
+template <class St, int EDGE>
+void ts_mode(cs_lattice* l, int k)
+{
+    if (l->has_flags) ts_coll<St, EDGE, MODE_REF>(l, k);
+    else ts_coll<St, EDGE, MODE_FLUID>(l, k);
+}
+
+template <class St>
+void ts_edge(cs_lattice* l, int k)
+{
+    if (l->params.edge == CS_EDGE_PERIODIC) ts_mode<St, CS_EDGE_PERIODIC>(l, k);
+    else ts_mode<St, CS_EDGE_ZERO>(l, k);
+}
+
+}  // namespace
+
+namespace cs {
+
+bool ts_takes(const cs_lattice* l)
+{
+    if (l->storage != CS_F32 && l->storage != CS_F32DEV) return false;
+    if (l->params.collision == CS_COLL_KBC) return false;
+    if (l->has_flags && l->params.boundary == CS_BB_HALFWAY) return false;
+    constexpr int K = 8, V = ts_cells<float>();
+    if (l->h < 2 * K) return false;  // the kernel wraps a row index once
+    const TsSplit s = ts_split(l, V, K);
+    // both waves of (nearly) every SIMD, or the region kernels' many small blocks win
+    if ((int64_t)s.strips * s.chunks < 6 * (int64_t)l->ctx->prop.multiProcessorCount) return false;
+    const double rows = (double)l->h / s.chunks;
+    const double stream = (double)s.strips * 64 * V * (rows + K - 1) / ((double)l->w * rows);
+    constexpr int IN = TB_EDGE - 2 * K;
+    const double regions = (double)((l->w + IN - 1) / IN) * ((l->h + IN - 1) / IN) * TB_EDGE * TB_EDGE /
+                           ((double)l->w * l->h);
+    return 1.12 * stream < regions;
+}
+
+void launch_ts(cs_lattice* l, int k)
+{
+    if (l->storage == CS_F32) ts_edge<StF32>(l, k);
+    else ts_edge<StF32Dev>(l, k);
+}
+
+}  // namespace cs

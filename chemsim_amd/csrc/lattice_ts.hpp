@@ -1,0 +1,57 @@
+// Launch of the streaming temporally blocked step kernel (lbm_ts.hpp), shared
+// by the units that instantiate it.
+#pragma once
+
+#include <algorithm>
+#include <type_traits>
+
+#include "cs_internal.hpp"
+#include "lbm_ts.hpp"
+
+namespace cs {
+
+// Columns per lane: two for 32-bit arithmetic.
+template <class T>
+constexpr int ts_cells() { return 2; }
+
+// Waves are independent and all resident at once, two per SIMD; rows are
+// split into as many runs as that allows, of at least 8 rows.
+struct TsSplit {
+    int strips, chunks;
+};
+inline TsSplit ts_split(const cs_lattice* l, int v, int k)
+{
+    const int in = 64 * v - 2 * k;
+    TsSplit s;
+    s.strips = (l->w + in - 1) / in;
+    const int waves = 2 * 4 * std::max(1, l->ctx->prop.multiProcessorCount);
+    s.chunks = std::clamp(waves / s.strips, 1, (l->h + 7) / 8);
+    return s;
+}
+
+template <class St, int EDGE, int MODE, int K, int COLL>
+void ts_launch(cs_lattice* l)
+{
+    using T = typename St::T;
+    constexpr int V = ts_cells<T>();
+    const TsSplit sp = ts_split(l, V, K);
+    TsArgs<T, K> A{};
+    A.a.fin = l->buf[l->cur];
+    A.a.fout = l->buf[l->cur ^ 1];
+    A.a.node = MODE == MODE_FLUID ? nullptr : l->node;
+    A.a.w = l->w;
+    A.a.h = l->h;
+    A.a.pitch = l->pitch;
+    A.a.cpitch = l->cpitch;
+    A.a.plane = l->plane;
+    A.a.k = l->k32;
+    A.strips = sp.strips;
+    A.chunks = sp.chunks;
+    const unsigned blocks = (unsigned)(((int64_t)A.strips * A.chunks + TS_WAVES - 1) / TS_WAVES);
+    hipLaunchKernelGGL((k_step_ts<St, EDGE, MODE, K, COLL, V, false>), dim3(blocks), dim3(TS_THREADS), 0, l->stream, A);
+    l->cur ^= 1;
+    l->steps += K;
+    for (int s = 0; s < K; ++s) l->time += l->params.delta_t;  // as step by step (lbm.rs:713)
+}
+
+}  // namespace cs

@@ -219,6 +219,98 @@ __device__ __forceinline__ float recip_rn<float>(float b)
     return 1.0f / b;
 }
 
+// The same value without the hardware reciprocal, for the kernels that have no
+// other instruction of its kind: v_rcp_f32, like the DPP moves, keeps the two waves
+// of a SIMD from issuing side by side for about a thousand cycles after it
+// (measured: add/mul streams of two waves 0.46 wave instructions per SIMD and
+// cycle, with one v_rcp_f32 in 256 instructions 0.26).  Newton-Raphson from
+// the integer estimate magic - bits(b) (within 6%): a cubic step, y (1 + e +
+// e^2) with e = 1 - b y, brings it to 2e-4, a quadratic one to an ulp, and the
+// last, y + y e with e exact, is the FMA reciprocal iteration of P. W.
+// Markstein, "Computation of elementary functions on the IBM RISC System/6000
+// processor", IBM J. Res. Dev. 34(1), 1990.  It misses the correctly rounded
+// value only where b's significand is all ones (e is then exactly 2^-24, which
+// `ok` excludes) and outside biased exponents 1 .. 251; all 2^32 inputs were
+// compared with the IEEE quotient (cs_check_reciprocal repeats that on the GPU
+// at hand).  Those inputs take the IEEE division, on a branch that only a wave
+// holding one enters.
+__device__ __forceinline__ float recip_newton(float b, bool& ok)
+{
+    const uint32_t x = __builtin_bit_cast(uint32_t, b);
+    float y = __builtin_bit_cast(float, 0x7EF311C7u - x);
+    float e = __builtin_fmaf(-b, y, 1.0f);
+    y = __builtin_fmaf(__builtin_fmaf(e, e, e), y, y);
+    e = __builtin_fmaf(-b, y, 1.0f);
+    y = __builtin_fmaf(e, y, y);
+    e = __builtin_fmaf(-b, y, 1.0f);
+    ok = ok && (x << 1) - 0x01000000u < 0xFB000000u && e != 0x1p-24f;
+    return __builtin_fmaf(e, y, y);
+}
+// V cells updated together, operation by operation.  A wave's dependent
+// instructions issue about 8 cycles apart, independent ones about 4.5, so the
+// collision functions below, instantiated with X = Cells<T, V>, alternate
+// between the cells where one cell's chain of sums would stall.
+template <class T, int V>
+struct Cells {
+    T v[V];
+    Cells() = default;
+    __device__ __forceinline__ explicit Cells(T x)
+    {
+#pragma unroll
+        for (int j = 0; j < V; ++j) v[j] = x;
+    }
+    __device__ __forceinline__ Cells operator-() const
+    {
+        Cells r;
+#pragma unroll
+        for (int j = 0; j < V; ++j) r.v[j] = -v[j];
+        return r;
+    }
+};
+#define CS_CELLS_OP(op)                                                                         \
+    template <class T, int V>                                                                   \
+    __device__ __forceinline__ Cells<T, V> operator op(const Cells<T, V>& a, const Cells<T, V>& b) \
+    {                                                                                           \
+        Cells<T, V> r;                                                                          \
+        _Pragma("unroll") for (int j = 0; j < V; ++j) r.v[j] = a.v[j] op b.v[j];                \
+        return r;                                                                               \
+    }                                                                                           \
+    template <class T, int V>                                                                   \
+    __device__ __forceinline__ Cells<T, V> operator op(const Cells<T, V>& a, std::type_identity_t<T> b) \
+    {                                                                                           \
+        Cells<T, V> r;                                                                          \
+        _Pragma("unroll") for (int j = 0; j < V; ++j) r.v[j] = a.v[j] op b;                     \
+        return r;                                                                               \
+    }                                                                                           \
+    template <class T, int V>                                                                   \
+    __device__ __forceinline__ Cells<T, V> operator op(std::type_identity_t<T> a, const Cells<T, V>& b) \
+    {                                                                                           \
+        Cells<T, V> r;                                                                          \
+        _Pragma("unroll") for (int j = 0; j < V; ++j) r.v[j] = a op b.v[j];                     \
+        return r;                                                                               \
+    }
+CS_CELLS_OP(+)
+CS_CELLS_OP(-)
+CS_CELLS_OP(*)
+CS_CELLS_OP(/)
+#undef CS_CELLS_OP
+// 1 / b of every cell, one branch for all of them.
+template <class T, int V>
+__device__ __forceinline__ Cells<T, V> recip_rn(const Cells<T, V>& b)
+{
+    Cells<T, V> r;
+    bool ok = std::is_same_v<T, float>;
+    if constexpr (std::is_same_v<T, float>) {
+#pragma unroll
+        for (int j = 0; j < V; ++j) r.v[j] = recip_newton(b.v[j], ok);
+    }
+    if (!ok) {
+#pragma unroll
+        for (int j = 0; j < V; ++j) r.v[j] = T(1) / b.v[j];
+    }
+    return r;
+}
+
 // ------------------------------------------------------------ cell update --
 // c_i . u for the nine directions, {0, ux, uy, -ux, -uy, ux + uy, -ux + uy,
 // -ux - uy, ux - uy} as the reference sums them.  The last two are written as
@@ -227,12 +319,12 @@ __device__ __forceinline__ float recip_rn<float>(float b)
 // (an exact zero may change sign, which 1 + vc A and vc vc, the only uses,
 // absorb), and the compiler then shares vc A, vc vc and (vc vc) B between
 // the opposite diagonals: 8 fewer operations per cell update.
-template <class T>
-__device__ __forceinline__ void lattice_dots(T ux, T uy, T (&vc)[9])
+template <class X>
+__device__ __forceinline__ void lattice_dots(X ux, X uy, X (&vc)[9])
 {
 #pragma clang fp contract(off)
-    const T d1 = ux + uy, d2 = -ux + uy;
-    vc[0] = T(0);
+    const X d1 = ux + uy, d2 = -ux + uy;
+    vc[0] = X(0);
     vc[1] = ux;
     vc[2] = uy;
     vc[3] = -ux;
@@ -243,25 +335,37 @@ __device__ __forceinline__ void lattice_dots(T ux, T uy, T (&vc)[9])
     vc[8] = -d2;
 }
 
+// The q-th direction that BGK finishes: for several cells at once 5 and 8
+// first, whose exchange between lanes the streaming kernel (lbm_ts.hpp) starts
+// meanwhile; 0 .. 8 for one cell (the region kernels measured 1% slower with
+// the other order).
+template <class T, class X>
+__device__ constexpr int nth_direction(int q)
+{
+    constexpr int PULL_FIRST[9] = {5, 8, 7, 6, 0, 1, 3, 2, 4};
+    return std::is_same_v<T, X> ? q : PULL_FIRST[q];
+}
+
 // Moments, equilibrium and BGK (lbm.rs:117-149, 43-71, 350-364) with the
 // reference's operation order; terms that multiply by a zero lattice
 // component are dropped, which leaves every value unchanged.
-template <class T>
-__device__ __forceinline__ void bgk_collide(const Consts<T>& k, T (&B)[9])
+template <class T, class X>
+__device__ __forceinline__ void bgk_collide(const Consts<T>& k, X (&B)[9])
 {
 #pragma clang fp contract(off)
-    const T rho = (((((((B[0] + B[1]) + B[2]) + B[3]) + B[4]) + B[5]) + B[6]) + B[7]) + B[8];
-    const T mx = ((((B[1] - B[3]) + B[5]) - B[6]) - B[7]) + B[8];
-    const T my = ((((B[2] - B[4]) + B[5]) + B[6]) - B[7]) - B[8];
-    const T inv = recip_rn(rho);
-    const T ux = inv * mx, uy = inv * my;
-    const T v2 = ux * ux + uy * uy;
-    T vc[9];
+    const X rho = (((((((B[0] + B[1]) + B[2]) + B[3]) + B[4]) + B[5]) + B[6]) + B[7]) + B[8];
+    const X mx = ((((B[1] - B[3]) + B[5]) - B[6]) - B[7]) + B[8];
+    const X my = ((((B[2] - B[4]) + B[5]) + B[6]) - B[7]) - B[8];
+    const X inv = recip_rn(rho);
+    const X ux = inv * mx, uy = inv * my;
+    const X v2 = ux * ux + uy * uy;
+    X vc[9];
     lattice_dots(ux, uy, vc);
 #pragma unroll
-    for (int i = 0; i < 9; ++i) {
-        const T s = ((T(1) + vc[i] * k.A) + (vc[i] * vc[i]) * k.B) + v2 * k.C;
-        const T feq = (rho * k.w(i)) * s;
+    for (int q = 0; q < 9; ++q) {
+        const int i = nth_direction<T, X>(q);
+        const X s = ((T(1) + vc[i] * k.A) + (vc[i] * vc[i]) * k.B) + v2 * k.C;
+        const X feq = (rho * k.w(i)) * s;
         B[i] = B[i] + (B[i] - feq) * k.K;
     }
 }
@@ -272,31 +376,31 @@ __device__ __forceinline__ void bgk_collide(const Consts<T>& k, T (&B)[9])
 // *populations* for i = 1..8 (lbm.rs:311-323), then
 //   omega_i = ((f+ - f_eq+) wp + (f- - f_eq-) wm) (-dt / 2),  f_i' = f_i + omega_i
 // with f+- = f_i +- f_sw_i and f_eq+- = f_eq_i +- f_eq_sw_i, in that order.
-template <class T>
-__device__ __forceinline__ void trt_collide(const Consts<T>& k, T (&B)[9])
+template <class T, class X>
+__device__ __forceinline__ void trt_collide(const Consts<T>& k, X (&B)[9])
 {
 #pragma clang fp contract(off)
-    const T rho = (((((((B[0] + B[1]) + B[2]) + B[3]) + B[4]) + B[5]) + B[6]) + B[7]) + B[8];
-    const T mx = ((((B[1] - B[3]) + B[5]) - B[6]) - B[7]) + B[8];
-    const T my = ((((B[2] - B[4]) + B[5]) + B[6]) - B[7]) - B[8];
-    const T inv = recip_rn(rho);
-    const T ux = inv * mx, uy = inv * my;
-    const T v2 = ux * ux + uy * uy;
-    T vc[9];
+    const X rho = (((((((B[0] + B[1]) + B[2]) + B[3]) + B[4]) + B[5]) + B[6]) + B[7]) + B[8];
+    const X mx = ((((B[1] - B[3]) + B[5]) - B[6]) - B[7]) + B[8];
+    const X my = ((((B[2] - B[4]) + B[5]) + B[6]) - B[7]) - B[8];
+    const X inv = recip_rn(rho);
+    const X ux = inv * mx, uy = inv * my;
+    const X v2 = ux * ux + uy * uy;
+    X vc[9];
     lattice_dots(ux, uy, vc);
-    T feq[9];
+    X feq[9];
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
-        const T s = ((T(1) + vc[i] * k.A) + (vc[i] * vc[i]) * k.B) + v2 * k.C;
+        const X s = ((T(1) + vc[i] * k.A) + (vc[i] * vc[i]) * k.B) + v2 * k.C;
         feq[i] = (rho * k.w(i)) * s;
     }
-    T o[9];
+    X o[9];
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
-        const T fsw = B[OPP[i]];
-        const T feqsw = i == 0 ? feq[0] : B[OPP[i]];
-        const T fp = B[i] + fsw, fm = B[i] - fsw;
-        const T feqp = feq[i] + feqsw, feqm = feq[i] - feqsw;
+        const X fsw = B[OPP[i]];
+        const X feqsw = i == 0 ? feq[0] : B[OPP[i]];
+        const X fp = B[i] + fsw, fm = B[i] - fsw;
+        const X feqp = feq[i] + feqsw, feqm = feq[i] - feqsw;
         o[i] = B[i] + ((fp - feqp) * k.wp + (fm - feqm) * k.wm) * k.hdt;
     }
 #pragma unroll
@@ -305,23 +409,23 @@ __device__ __forceinline__ void trt_collide(const Consts<T>& k, T (&B)[9])
 
 // Moments and equilibrium of one cell as Lattice::equilibrium computes them
 // (lbm.rs:117-160, 43-71).
-template <class T>
-__device__ __forceinline__ void cell_equilibrium(const Consts<T>& k, const T (&B)[9], T& rho, T& ux, T& uy,
-                                                 T (&feq)[9])
+template <class T, class X>
+__device__ __forceinline__ void cell_equilibrium(const Consts<T>& k, const X (&B)[9], X& rho, X& ux, X& uy,
+                                                 X (&feq)[9])
 {
 #pragma clang fp contract(off)
     rho = (((((((B[0] + B[1]) + B[2]) + B[3]) + B[4]) + B[5]) + B[6]) + B[7]) + B[8];
-    const T mx = ((((B[1] - B[3]) + B[5]) - B[6]) - B[7]) + B[8];
-    const T my = ((((B[2] - B[4]) + B[5]) + B[6]) - B[7]) - B[8];
-    const T inv = recip_rn(rho);
+    const X mx = ((((B[1] - B[3]) + B[5]) - B[6]) - B[7]) + B[8];
+    const X my = ((((B[2] - B[4]) + B[5]) + B[6]) - B[7]) - B[8];
+    const X inv = recip_rn(rho);
     ux = inv * mx;
     uy = inv * my;
-    const T v2 = ux * ux + uy * uy;
-    T vc[9];
+    const X v2 = ux * ux + uy * uy;
+    X vc[9];
     lattice_dots(ux, uy, vc);
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
-        const T s = ((T(1) + vc[i] * k.A) + (vc[i] * vc[i]) * k.B) + v2 * k.C;
+        const X s = ((T(1) + vc[i] * k.A) + (vc[i] * vc[i]) * k.B) + v2 * k.C;
         feq[i] = (rho * k.w(i)) * s;
     }
 }
@@ -331,16 +435,16 @@ __device__ __forceinline__ void cell_equilibrium(const Consts<T>& k, const T (&B
 //   P_ab = sum_i f_neq_i c_ia c_ib,  Q_i,ab = c_ia c_ib - cs^2 delta_ab,
 //   reg_i = (((f_eq_i + P_xx (Q_xx sf)) + P_xy (Q_xy sf)) + P_yx (Q_yx sf)) + P_yy (Q_yy sf),
 // sf = w_i / (2 cs^4).  The wrapped operator is never called (as in the reference).
-template <class T>
-__device__ __forceinline__ void reg_collide(const Consts<T>& k, T (&B)[9])
+template <class T, class X>
+__device__ __forceinline__ void reg_collide(const Consts<T>& k, X (&B)[9])
 {
 #pragma clang fp contract(off)
-    T rho, ux, uy, feq[9];
+    X rho, ux, uy, feq[9];
     cell_equilibrium(k, B, rho, ux, uy, feq);
-    T pxx = T(0), pxy = T(0), pyx = T(0), pyy = T(0);
+    X pxx = X(0), pxy = X(0), pyx = X(0), pyy = X(0);
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
-        const T fneq = B[i] - feq[i];
+        const X fneq = B[i] - feq[i];
         const T cx = T(CX[i]), cy = T(CY[i]);
         pxx = pxx + fneq * (cx * cx);
         pxy = pxy + fneq * (cx * cy);
@@ -351,7 +455,7 @@ __device__ __forceinline__ void reg_collide(const Consts<T>& k, T (&B)[9])
     for (int i = 0; i < 9; ++i) {
         const T cx = T(CX[i]), cy = T(CY[i]);
         const T sf = k.sfq[Consts<T>::wclass(i)];
-        T reg = feq[i];
+        X reg = feq[i];
         reg = reg + pxx * ((cx * cx - k.cs2) * sf);
         reg = reg + pxy * ((cx * cy) * sf);
         reg = reg + pyx * ((cy * cx) * sf);
@@ -370,29 +474,29 @@ __device__ __forceinline__ void reg_collide(const Consts<T>& k, T (&B)[9])
 //   dh_i = (f_i - f_eq_i) - ds_i,
 //   gamma = -(((sum ds dh / f_eq) / (sum dh dh / f_eq)) (2 - 1/beta) + (-1/beta)),
 //   f_i' = f_i + (ds_i (2 (-beta)) + (dh_i gamma) (-beta)).
-template <class T>
-__device__ __forceinline__ void kbc_collide(const Consts<T>& k, T (&B)[9])
+template <class T, class X>
+__device__ __forceinline__ void kbc_collide(const Consts<T>& k, X (&B)[9])
 {
 #pragma clang fp contract(off)
-    T rho, u, v, feq[9];
+    X rho, u, v, feq[9];
     cell_equilibrium(k, B, rho, u, v, feq);
     const T dx = k.dx;
-    const T uv = u * v, u2 = u * u, v2 = v * v;
+    const X uv = u * v, u2 = u * u, v2 = v * v;
     const T dx2 = dx * dx;
-    T temp = T(0);
+    X temp = X(0);
 #pragma unroll
     for (int i = 0; i < 9; ++i) temp = temp + B[i] * dx2;
-    const T pit = temp - uv;
-    const T nt = v2 - u2;
-    const T uv8 = uv * T(8);
-    const T ds0 = (((uv8 * pit) + nt * nt) * rho) * T(0.5);
-    const T ds13 = (((((u * dx - nt) + T(1)) * nt) - ((v * (dx * T(4))) + uv8) * pit) * rho) * T(0.25);
-    const T ds24 = (((((v * (-dx) - nt) + T(-1)) * nt) - ((u * (dx * T(4))) + uv8) * pit) * rho) * T(0.25);
-    const T ds58 = (((((uv8 + u * (T(4) * dx)) + (T(2) * dx) * dx) * pit) + ((nt - (v - u) * dx) * nt)) * rho) *
+    const X pit = temp - uv;
+    const X nt = v2 - u2;
+    const X uv8 = uv * T(8);
+    const X ds0 = (((uv8 * pit) + nt * nt) * rho) * T(0.5);
+    const X ds13 = (((((u * dx - nt) + T(1)) * nt) - ((v * (dx * T(4))) + uv8) * pit) * rho) * T(0.25);
+    const X ds24 = (((((v * (-dx) - nt) + T(-1)) * nt) - ((u * (dx * T(4))) + uv8) * pit) * rho) * T(0.25);
+    const X ds58 = (((((uv8 + u * (T(4) * dx)) + (T(2) * dx) * dx) * pit) + ((nt - (v - u) * dx) * nt)) * rho) *
                    T(0.125);
-    const T ds[9] = {ds0, ds13, ds24, ds13, ds24, ds58, ds58, ds58, ds58};
-    T dh[9];
-    T num = T(0), den = T(0);
+    const X ds[9] = {ds0, ds13, ds24, ds13, ds24, ds58, ds58, ds58, ds58};
+    X dh[9];
+    X num = X(0), den = X(0);
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
         dh[i] = (B[i] - feq[i]) - ds[i];
@@ -400,7 +504,7 @@ __device__ __forceinline__ void kbc_collide(const Consts<T>& k, T (&B)[9])
         den = den + (dh[i] * dh[i]) / feq[i];
     }
     const T beta = k.beta;
-    const T gamma = (((num / den) * (T(2) - T(1) / beta)) + (-T(1) / beta)) * T(-1);
+    const X gamma = (((num / den) * (T(2) - T(1) / beta)) + (-T(1) / beta)) * T(-1);
     const T m2b = T(2) * (-beta);
 #pragma unroll
     for (int i = 0; i < 9; ++i) B[i] = B[i] + (ds[i] * m2b + (dh[i] * gamma) * (-beta));
@@ -411,23 +515,24 @@ __device__ __forceinline__ void kbc_collide(const Consts<T>& k, T (&B)[9])
 //   g_eq_i = w_i (drho + rho ((vc A + vc^2 B) + v2 C)),  g'_i = g_i + (g_i - g_eq_i) K,
 // the same BGK update as bgk_collide without carrying the O(1) rest
 // populations through the rounding.
-template <class T>
-__device__ __forceinline__ void bgk_collide_dev(const Consts<T>& k, T (&B)[9])
+template <class T, class X>
+__device__ __forceinline__ void bgk_collide_dev(const Consts<T>& k, X (&B)[9])
 {
 #pragma clang fp contract(off)
-    const T drho = (((((((B[0] + B[1]) + B[2]) + B[3]) + B[4]) + B[5]) + B[6]) + B[7]) + B[8];
-    const T rho = k.rho0 + drho;
-    const T mx = ((((B[1] - B[3]) + B[5]) - B[6]) - B[7]) + B[8];
-    const T my = ((((B[2] - B[4]) + B[5]) + B[6]) - B[7]) - B[8];
-    const T inv = recip_rn(rho);
-    const T ux = inv * mx, uy = inv * my;
-    const T v2 = ux * ux + uy * uy;
-    T vc[9];
+    const X drho = (((((((B[0] + B[1]) + B[2]) + B[3]) + B[4]) + B[5]) + B[6]) + B[7]) + B[8];
+    const X rho = k.rho0 + drho;
+    const X mx = ((((B[1] - B[3]) + B[5]) - B[6]) - B[7]) + B[8];
+    const X my = ((((B[2] - B[4]) + B[5]) + B[6]) - B[7]) - B[8];
+    const X inv = recip_rn(rho);
+    const X ux = inv * mx, uy = inv * my;
+    const X v2 = ux * ux + uy * uy;
+    X vc[9];
     lattice_dots(ux, uy, vc);
 #pragma unroll
-    for (int i = 0; i < 9; ++i) {
-        const T s = (vc[i] * k.A + (vc[i] * vc[i]) * k.B) + v2 * k.C;
-        const T geq = k.w(i) * (drho + rho * s);
+    for (int q = 0; q < 9; ++q) {
+        const int i = nth_direction<T, X>(q);
+        const X s = (vc[i] * k.A + (vc[i] * vc[i]) * k.B) + v2 * k.C;
+        const X geq = k.w(i) * (drho + rho * s);
         B[i] = B[i] + (B[i] - geq) * k.K;
     }
 }

@@ -41,8 +41,8 @@ constexpr int TB_SLOTS = TB_EDGE * TB_EDGE / TB_THREADS;
 constexpr int TB_EDGE_SMALL = 32;
 
 // Collision of one fluid cell: the operator finish() applies.
-template <class St, int COLL>
-__device__ __forceinline__ void collide_cell(const Consts<typename St::T>& k, typename St::T (&B)[9])
+template <class St, int COLL, class X>
+__device__ __forceinline__ void collide_cell(const Consts<typename St::T>& k, X (&B)[9])
 {
     if constexpr (COLL != CS_COLL_BGK) static_assert(!St::DEV, "TRT, Regularized and KBC run in the reference arithmetic");
     if constexpr (COLL == CS_COLL_TRT) trt_collide(k, B);

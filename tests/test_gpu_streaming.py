@@ -1,0 +1,78 @@
+"""The streaming temporally blocked step (k_step_ts) against the CPU oracle,
+value for value, on lattices that the built-in choice gives to it: one strip
+and very many rows, very wide and flat, and ragged in both directions; zero
+and periodic edges; the reference's solid mask; every operator it runs; steps
+that leave a 4-step launch and single steps over."""
+import numpy as np
+import pytest
+
+from chemsim_amd import Lattice, capi
+from oracle import pyoracle as O
+from test_gpu_temporal import OPERATORS, gpu_params, rand_state, random_flags
+
+pytestmark = pytest.mark.gpu
+
+# (w, h): a part strip; 18 strips of ragged width; a run of rows per wave with one column over
+SHAPES = [(101, 30011), (2003, 2300), (24641, 163)]
+
+
+@pytest.mark.parametrize("edge", [O.EDGE_ZERO, O.EDGE_PERIODIC])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("shape", SHAPES, ids=[f"{w}x{h}" for w, h in SHAPES])
+def test_bgk_matches_oracle(ctx, shape, masked, edge):
+    w, h = shape
+    rng = np.random.default_rng(61)
+    f = rand_state(rng, h, w)
+    flags = random_flags(rng, h, w) if masked else None
+    if masked:
+        flags[:, w // 3:] = 0  # strips and rows with and without solid cells
+        flags[h // 2:] = 0
+    op = O.params(w, h, tau=0.62, edge=edge)
+    with Lattice(ctx, w, h, "f32", gpu_params(op), flags) as lat:
+        assert lat.temporal_steps() == 8
+        lat.upload(f)
+        lat.step(21)  # two 8-step launches, one of 4, one step
+        np.testing.assert_array_equal(lat.download(), O.run(op, f, 21, flags))
+
+
+@pytest.mark.parametrize("coll", ["trt", "regularized"])
+def test_operators_match_oracle(ctx, coll):
+    w, h = SHAPES[1]
+    rng = np.random.default_rng(62)
+    f = rand_state(rng, h, w)
+    flags = random_flags(rng, h, w)
+    flags[:, w // 2:] = 0
+    op = O.params(w, h, edge=O.EDGE_PERIODIC, **OPERATORS[coll])
+    with Lattice(ctx, w, h, "f32", gpu_params(op), flags) as lat:
+        lat.upload(f)
+        lat.step(9)
+        np.testing.assert_array_equal(lat.download(), O.run(op, f, 9, flags))
+
+
+@pytest.mark.parametrize("edge", [O.EDGE_ZERO, O.EDGE_PERIODIC])
+def test_deviations_match_oracle(ctx, edge):
+    w, h = SHAPES[1]
+    rng = np.random.default_rng(63)
+    op = O.params(w, h, tau=0.7, edge=edge)
+    rho = (1 + 0.01 * rng.standard_normal((h, w))).astype(np.float32)
+    u = (0.03 * rng.standard_normal((2, h, w))).astype(np.float32)
+    with Lattice(ctx, w, h, "f32dev", gpu_params(op)) as lat:
+        lat.init_equilibrium(rho, u[0], u[1])
+        lat.step(12)
+        np.testing.assert_array_equal(lat.download_raw(), O.run_devf32(op, O.equilibrium_dev(op, rho, u[0], u[1]), 12))
+
+
+def test_unusual_densities_match_oracle(ctx):
+    """Densities that take the reciprocal's IEEE branch: zero, subnormal, huge
+    and all-ones significands beside ordinary ones."""
+    w, h = SHAPES[1]
+    rng = np.random.default_rng(64)
+    f = rand_state(rng, h, w)
+    for k, v in enumerate([0.0, 1e-40, 3e37, 2.0 - 2.0 ** -23]):
+        f[:, 100 + 40 * k:110 + 40 * k, 200:230] = 0
+        f[0, 100 + 40 * k:110 + 40 * k, 200:230] = v
+    op = O.params(w, h, tau=0.8, edge=O.EDGE_PERIODIC)
+    with Lattice(ctx, w, h, "f32", gpu_params(op)) as lat:
+        lat.upload(f)
+        lat.step(8)
+        np.testing.assert_array_equal(lat.download(), O.run(op, f, 8))
