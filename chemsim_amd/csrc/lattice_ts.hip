@@ -11,6 +11,14 @@
 // cells at 1536^2 .. 8192^2 is 1.07 .. 1.14).  FP32 Taylor-Green, GLUPS,
 // streaming / regions in registers: 1024^2 110 / 174, 1536^2 187 / 218,
 // 2048^2 198 / 194, 3072^2 263 / 228, 4096^2 306 / 242, 8192^2 350 / 254.
+//
+// FP64 has no region kernels (a region would not fit), and its one-step kernel
+// is bound by HBM at 144 bytes per cell update: GLUPS, streaming / one-step,
+// 512^2 50 / 35, 1024^2 92 / 39, 2048^2 126 / 40, 4096^2 162 / 43, half-way
+// cavity 2048^2 82 / 38.  Lattices of 2^20 cells on take it; below that
+// cs_lattice_temporal_steps goes on reporting one step per launch.  KBC keeps
+// the one-step kernel: its 19 divisions per cell already take as long as the
+// memory, and the strips' recomputation would add to them.
 #include "lattice_ts.hpp"
 #include "lbm_tb.hpp"
 
@@ -58,11 +66,12 @@ namespace cs {
 
 bool ts_takes(const cs_lattice* l)
 {
-    if (l->storage != CS_F32 && l->storage != CS_F32DEV) return false;
-    if (l->params.collision == CS_COLL_KBC) return false;
-    if (l->has_flags && l->params.boundary == CS_BB_HALFWAY) return false;
     constexpr int K = 8, V = ts_cells<float>();
+    if (l->params.collision == CS_COLL_KBC) return false;
     if (l->h < 2 * K) return false;  // the kernel wraps a row index once
+    if (l->storage == CS_F64) return (int64_t)l->w * l->h >= (int64_t)1 << 20;
+    if (l->storage != CS_F32 && l->storage != CS_F32DEV) return false;
+    if (l->has_flags && l->params.boundary == CS_BB_HALFWAY) return false;
     const TsSplit s = ts_split(l, V, K);
     // both waves of (nearly) every SIMD, or the region kernels' many small blocks win
     if ((int64_t)s.strips * s.chunks < 6 * (int64_t)l->ctx->prop.multiProcessorCount) return false;
@@ -76,7 +85,8 @@ bool ts_takes(const cs_lattice* l)
 
 void launch_ts(cs_lattice* l, int k)
 {
-    if (l->storage == CS_F32) ts_edge<StF32>(l, k);
+    if (l->storage == CS_F64) launch_ts_f64(l, k);
+    else if (l->storage == CS_F32) ts_edge<StF32>(l, k);
     else ts_edge<StF32Dev>(l, k);
 }
 

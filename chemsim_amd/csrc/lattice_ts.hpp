@@ -10,9 +10,10 @@
 
 namespace cs {
 
-// Columns per lane: two for 32-bit arithmetic.
+// Columns per lane: two for 32-bit arithmetic, one for 64-bit (the kept rows of
+// 8 levels take the same registers).
 template <class T>
-constexpr int ts_cells() { return 2; }
+constexpr int ts_cells() { return sizeof(T) == 8 ? 1 : 2; }
 
 // Waves are independent and all resident at once, two per SIMD; rows are
 // split into as many runs as that allows, of at least 8 rows.
@@ -44,7 +45,8 @@ void ts_launch(cs_lattice* l)
     A.a.pitch = l->pitch;
     A.a.cpitch = l->cpitch;
     A.a.plane = l->plane;
-    A.a.k = l->k32;
+    if constexpr (std::is_same_v<T, double>) A.a.k = l->k64;
+    else A.a.k = l->k32;
     A.strips = sp.strips;
     A.chunks = sp.chunks;
     const unsigned blocks = (unsigned)(((int64_t)A.strips * A.chunks + TS_WAVES - 1) / TS_WAVES);
@@ -53,5 +55,8 @@ void ts_launch(cs_lattice* l)
     l->steps += K;
     for (int s = 0; s < K; ++s) l->time += l->params.delta_t;  // as step by step (lbm.rs:713)
 }
+
+// The unit that instantiates it per storage: k = 8 or, for BGK, 4 steps.
+void launch_ts_f64(cs_lattice* l, int k);
 
 }  // namespace cs

@@ -6,7 +6,8 @@ that leave a 4-step launch and single steps over."""
 import numpy as np
 import pytest
 
-from chemsim_amd import Lattice, capi
+from chemsim_amd import Lattice, Params, capi
+from chemsim_amd import workloads as W
 from oracle import pyoracle as O
 from test_gpu_temporal import OPERATORS, gpu_params, rand_state, random_flags
 
@@ -76,3 +77,57 @@ def test_unusual_densities_match_oracle(ctx):
         lat.upload(f)
         lat.step(8)
         np.testing.assert_array_equal(lat.download(), O.run(op, f, 8))
+
+
+F64_SHAPES = [(1100, 1001), (49, 22001), (65601, 17)]
+
+
+@pytest.mark.parametrize("edge", [O.EDGE_ZERO, O.EDGE_PERIODIC])
+@pytest.mark.parametrize("mode", ["fluid", "reference", "halfway"])
+@pytest.mark.parametrize("shape", F64_SHAPES, ids=[f"{w}x{h}" for w, h in F64_SHAPES])
+def test_f64_matches_oracle(ctx, shape, mode, edge):
+    w, h = shape
+    rng = np.random.default_rng(65)
+    f = rand_state(rng, h, w).astype(np.float64)
+    flags = None
+    if mode != "fluid":
+        flags = random_flags(rng, h, w)
+        flags[:, w // 2:] = 0
+        flags[h // 2:] = 0
+    kw = dict(boundary=O.BB_HALFWAY, lid=(0.02, -0.03)) if mode == "halfway" else {}
+    op = O.params(w, h, tau=0.62, edge=edge, **kw)
+    with Lattice(ctx, w, h, "f64", gpu_params(op), flags) as lat:
+        assert lat.temporal_steps() == 8
+        lat.upload(f)
+        lat.step(13)  # 8 steps, 4 steps, one step
+        np.testing.assert_array_equal(lat.download(np.float64), O.run(op, f, 13, flags))
+
+
+@pytest.mark.parametrize("coll", ["trt", "regularized"])
+def test_f64_operators_match_oracle(ctx, coll):
+    w, h = F64_SHAPES[0]
+    rng = np.random.default_rng(66)
+    f = rand_state(rng, h, w).astype(np.float64)
+    op = O.params(w, h, edge=O.EDGE_ZERO, **OPERATORS[coll])
+    with Lattice(ctx, w, h, "f64", gpu_params(op)) as lat:
+        lat.upload(f)
+        lat.step(8)
+        np.testing.assert_array_equal(lat.download(np.float64), O.run(op, f, 8))
+
+
+def test_f64_channel_matches_one_step(ctx):
+    """Inlet, outlet, obstacle and walls: eight steps in one launch equal eight
+    one-step launches."""
+    ch = W.Channel(w=2100, h=512, circles=[(200, 700, 60)], re=60.0, u_in=0.05)
+    p = Params(tau=ch.tau, boundary=capi.CS_BB_HALFWAY, inlet_uy=ch.u_in, outlet_rho=1.0)
+    out = []
+    try:
+        for k in (capi.CS_TEMPORAL_AUTO, 0):
+            capi.call("cs_set_temporal_steps", k)
+            with Lattice(ctx, ch.w, ch.h, "f64", p, ch.flags()) as lat:
+                lat.init_equilibrium(*[a.astype(np.float64) for a in W.rest_state(ch.w, ch.h)])
+                lat.step(24)
+                out.append(lat.download(np.float64))
+    finally:
+        capi.call("cs_set_temporal_steps", capi.CS_TEMPORAL_AUTO)
+    np.testing.assert_array_equal(out[0], out[1])
