@@ -134,7 +134,7 @@ int tb_steps(const cs_lattice* l, int cpt_override)
 {
     const int k = g_tb_steps.load(std::memory_order_relaxed);
     if (k == 0 || cpt_override != 0) return 0;
-    if (k == CS_TEMPORAL_AUTO && l->storage == CS_F64 && ts_takes(l)) return tb_plan(8, TS_PLAN);
+    if (k == CS_TEMPORAL_AUTO && storage_bytes(l->storage) != 4 && ts_takes(l)) return tb_plan(8, TS_PLAN);
     if (l->storage != CS_F32 && l->storage != CS_F32DEV) return 0;
     if ((int64_t)l->h * l->pitch * 4 >= ((int64_t)1 << 32)) return 0;  // 32-bit offsets
     if (k == CS_TEMPORAL_AUTO) {
@@ -151,6 +151,7 @@ int tb_steps(const cs_lattice* l, int cpt_override)
 
 int tb_remainder_plan(const cs_lattice* l, int plan)
 {
+    if (storage_bytes(l->storage) == 2) return 0;
     if (tb_plan_steps(plan) != 8 || l->params.collision != CS_COLL_BGK) return 0;
     return (plan & ~0xFF) | 4;
 }
@@ -181,4 +182,5 @@ extern "C" int cs_set_temporal_steps(int k)
 #ifndef CS_TS_UNITS
 #include "lattice_ts.hip"
 #include "lattice_ts_f64.hip"
+#include "lattice_ts_16.hip"
 #endif

@@ -19,6 +19,16 @@
 // cs_lattice_temporal_steps goes on reporting one step per launch.  KBC keeps
 // the one-step kernel: its 19 divisions per cell already take as long as the
 // memory, and the strips' recomputation would add to them.
+//
+// 16-bit storage rounds every level to 16 bits.  Against the one-step kernel
+// (computed cells per kept cell 1.94 at 1536^2, 1.62 at 2048^2, 1.36 at 3072^2,
+// 1.27 at 4096^2), GLUPS streaming / one-step:
+//   f16 to nearest 165 / 118, 186 / 131, 243 / 144, 268 / 153
+//   bf16 to nearest 131 / 110, 150 / 118, 194 / 140, 219 / 150
+//   bf16 stochastic 114 / 111, 130 / 121, 170 / 140, 191 / 150
+//   f16 stochastic 97 / 111, 117 / 118, 150 / 140, 161 / 150
+// so f16 with stochastic rounding takes it only where the fill is small.
+// Half-way walls keep the one-step kernel (f16 cavity 4096^2 103 / 115).
 #include "lattice_ts.hpp"
 #include "lbm_tb.hpp"
 
@@ -70,13 +80,16 @@ bool ts_takes(const cs_lattice* l)
     if (l->params.collision == CS_COLL_KBC) return false;
     if (l->h < 2 * K) return false;  // the kernel wraps a row index once
     if (l->storage == CS_F64) return (int64_t)l->w * l->h >= (int64_t)1 << 20;
-    if (l->storage != CS_F32 && l->storage != CS_F32DEV) return false;
     if (l->has_flags && l->params.boundary == CS_BB_HALFWAY) return false;
     const TsSplit s = ts_split(l, V, K);
     // both waves of (nearly) every SIMD, or the region kernels' many small blocks win
     if ((int64_t)s.strips * s.chunks < 6 * (int64_t)l->ctx->prop.multiProcessorCount) return false;
     const double rows = (double)l->h / s.chunks;
     const double stream = (double)s.strips * 64 * V * (rows + K - 1) / ((double)l->w * rows);
+    if (storage_bytes(l->storage) == 2) {
+        const bool sr = l->params.rounding == CS_ROUND_STOCHASTIC;
+        return stream < (!sr ? 2.2 : l->storage == CS_BF16DEV ? 1.9 : 1.45);
+    }
     constexpr int IN = TB_EDGE - 2 * K;
     const double regions = (double)((l->w + IN - 1) / IN) * ((l->h + IN - 1) / IN) * TB_EDGE * TB_EDGE /
                            ((double)l->w * l->h);
@@ -86,6 +99,7 @@ bool ts_takes(const cs_lattice* l)
 void launch_ts(cs_lattice* l, int k)
 {
     if (l->storage == CS_F64) launch_ts_f64(l, k);
+    else if (storage_bytes(l->storage) == 2) launch_ts_16(l);
     else if (l->storage == CS_F32) ts_edge<StF32>(l, k);
     else ts_edge<StF32Dev>(l, k);
 }

@@ -30,7 +30,7 @@ inline TsSplit ts_split(const cs_lattice* l, int v, int k)
     return s;
 }
 
-template <class St, int EDGE, int MODE, int K, int COLL>
+template <class St, int EDGE, int MODE, int K, int COLL, bool SR = false>
 void ts_launch(cs_lattice* l)
 {
     using T = typename St::T;
@@ -49,14 +49,17 @@ void ts_launch(cs_lattice* l)
     else A.a.k = l->k32;
     A.strips = sp.strips;
     A.chunks = sp.chunks;
+    if constexpr (SR)
+        for (int s = 0; s < K; ++s) A.keys[s] = sr_key(l->params.seed, l->steps + (uint64_t)s);
     const unsigned blocks = (unsigned)(((int64_t)A.strips * A.chunks + TS_WAVES - 1) / TS_WAVES);
-    hipLaunchKernelGGL((k_step_ts<St, EDGE, MODE, K, COLL, V, false>), dim3(blocks), dim3(TS_THREADS), 0, l->stream, A);
+    hipLaunchKernelGGL((k_step_ts<St, EDGE, MODE, K, COLL, V, SR>), dim3(blocks), dim3(TS_THREADS), 0, l->stream, A);
     l->cur ^= 1;
     l->steps += K;
     for (int s = 0; s < K; ++s) l->time += l->params.delta_t;  // as step by step (lbm.rs:713)
 }
 
-// The unit that instantiates it per storage: k = 8 or, for BGK, 4 steps.
+// The units that instantiate it per storage: k = 8 or, for BGK, 4 steps.
 void launch_ts_f64(cs_lattice* l, int k);
+void launch_ts_16(cs_lattice* l);  // 8 steps
 
 }  // namespace cs

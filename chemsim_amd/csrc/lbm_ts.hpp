@@ -72,6 +72,40 @@ __device__ __forceinline__ void ts_shift(const T (&x)[V], T e, T (&y)[V])
     for (int j = 0; j < V; ++j) y[j] = NEXT ? (j + 1 < V ? x[j + 1 < V ? j + 1 : 0] : e) : (j > 0 ? x[j > 0 ? j - 1 : 0] : e);
 }
 
+// The nine values of a cell rounded to the 16-bit storage, with finish()'s
+// random bits if SR.  For bf16 in the integer form (round to nearest even, or
+// the top 16 random bits added below the kept ones and truncated): the
+// conversions' NaN tests per value and v_cvt_sr_bf16_f32, which holds the
+// SIMD's second wave back (recip_newton's comment), cost more -- 4096^2
+// Taylor-Green, bf16 168 GLUPS to nearest and 157 stochastic with them.  A NaN
+// takes them.  For f16, whose subnormal results would need more instructions
+// than the conversion costs, the conversion itself.
+template <class St, bool SR>
+__device__ __forceinline__ void ts_round(float (&x)[9], uint32_t cell_key)
+{
+    uint32_t h = SR ? lowbias32(cell_key) : 0u;
+    if constexpr (std::is_same_v<St, StBF16>) {
+        bool nan = x[8] != x[8];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) nan = nan || __builtin_isunordered(x[2 * q], x[2 * q + 1]);
+        if (!nan) {
+#pragma unroll
+            for (int i = 0; i < 9; ++i) {
+                const uint32_t u = __builtin_bit_cast(uint32_t, x[i]);
+                const uint32_t add = !SR ? 0x7fffu + ((u >> 16) & 1u) : (i & 1) ? (h & 0xffffu) : (h >> 16);
+                x[i] = __builtin_bit_cast(float, (u + add) & 0xffff0000u);
+                if (SR && (i & 1)) h = xorshift32(h);
+            }
+            return;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        x[i] = St::wid(SR ? St::nar_sr(x[i], (i & 1) ? h << 16 : h) : St::nar(x[i]));
+        if (SR && (i & 1)) h = xorshift32(h);
+    }
+}
+
 // Per-wave LDS of the geometry modes.
 template <class T, int MODE, int K, int V>
 struct TsLds {
@@ -339,21 +373,9 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
                 // every step's result is rounded to the storage type, as a store would
 #pragma unroll
                 for (int j = 0; j < V; ++j) {
-                    if constexpr (SR) {
-                        bool in;
-                        const uint32_t g = (uint32_t)wrap_row(r, in);
-                        uint32_t h = lowbias32((a.cell_base + g * (uint32_t)a.w + col[j]) ^ A.keys[s - 1]);
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            C[j][2 * q] = St::wid(St::nar_sr(C[j][2 * q], h));
-                            C[j][2 * q + 1] = St::wid(St::nar_sr(C[j][2 * q + 1], h << 16));
-                            h = xorshift32(h);
-                        }
-                        C[j][8] = St::wid(St::nar_sr(C[j][8], h));
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < 9; ++i) C[j][i] = St::wid(St::nar(C[j][i]));
-                    }
+                    bool in;
+                    const uint32_t g = (uint32_t)wrap_row(r, in);
+                    ts_round<St, SR>(C[j], SR ? (a.cell_base + g * (uint32_t)a.w + col[j]) ^ A.keys[s - 1] : 0u);
                 }
             }
             if constexpr (HALF) {

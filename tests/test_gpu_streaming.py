@@ -131,3 +131,37 @@ def test_f64_channel_matches_one_step(ctx):
     finally:
         capi.call("cs_set_temporal_steps", capi.CS_TEMPORAL_AUTO)
     np.testing.assert_array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("edge", [O.EDGE_ZERO, O.EDGE_PERIODIC])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("rounding", [capi.CS_ROUND_NEAREST, capi.CS_ROUND_STOCHASTIC], ids=["nearest", "stochastic"])
+@pytest.mark.parametrize("storage", ["bf16", "f16"])
+def test_16bit_matches_one_step(ctx, storage, rounding, masked, edge):
+    """Every stored value, NaNs and infinities included, of 21 steps (two 8-step
+    launches and five single ones) against 21 one-step launches.  A NaN's sign
+    and payload are not compared: the one-step kernels with 1 and with 4 cells
+    per lane already differ in them."""
+    w, h = 3001, 3003
+    rng = np.random.default_rng(67)
+    rho = (1 + 0.01 * rng.standard_normal((h, w))).astype(np.float32)
+    u = (0.03 * rng.standard_normal((2, h, w))).astype(np.float32)
+    rho[1000, 1000], rho[2000, 50] = np.nan, 1e8
+    flags = random_flags(rng, h, w) if masked else None
+    if masked:
+        flags[:, w // 3:] = 0
+    p = Params(tau=0.7, edge=edge, rounding=rounding, seed=9)
+    out = []
+    try:
+        for k in (capi.CS_TEMPORAL_AUTO, 0):
+            capi.call("cs_set_temporal_steps", k)
+            with Lattice(ctx, w, h, storage, p, flags) as lat:
+                assert lat.temporal_steps() == (1 if k == 0 else 8)
+                lat.init_equilibrium(rho, u[0], u[1])
+                lat.step(21)
+                raw = lat.download_raw()
+                nan = np.uint16(0x7FC0 if storage == "bf16" else 0x7E00)
+                out.append(np.where((raw & 0x7FFF) > (0x7F80 if storage == "bf16" else 0x7C00), nan, raw))
+    finally:
+        capi.call("cs_set_temporal_steps", capi.CS_TEMPORAL_AUTO)
+    np.testing.assert_array_equal(out[0], out[1])
