@@ -481,6 +481,7 @@ struct cs_batch {
     std::vector<unsigned char> host_lats;  // BatchLat<T> descriptors
     std::vector<LatState> host_state;     // `state` as of the launch
     cs_batch_tuning tuning{256, 2, 1, CS_ORDER_LARGEST_FIRST, CS_LAUNCH_PERSISTENT};
+    KeptStaging staging;              // result planes of the moment calls
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
@@ -1031,7 +1032,8 @@ extern "C" int cs_batch_destroy(cs_batch* b)
         if (!b) return;
         if (b->stream) (void)hipStreamSynchronize(b->stream);
         for (void* p : {b->arena, (void*)b->nodes, b->d_lats, (void*)b->d_order, (void*)b->d_queue, (void*)b->snap,
-                        (void*)b->d_res, (void*)b->d_tiles, (void*)b->d_regions, (void*)b->d_bar, (void*)b->d_state})
+                        (void*)b->d_res, (void*)b->d_tiles, (void*)b->d_regions, (void*)b->d_bar, (void*)b->d_state,
+                        b->staging.p})
             if (p) (void)hipFree(p);
         if (b->ev0) (void)hipEventDestroy(b->ev0);
         if (b->ev1) (void)hipEventDestroy(b->ev1);
@@ -1194,34 +1196,33 @@ extern "C" int cs_batch_download_raw(cs_batch* b, int index, void* data)
     });
 }
 
+// k_moments of one lattice, planes in mask bit order copied to the caller's arrays.
+static void batch_moments(cs_batch* b, int index, unsigned mask, std::initializer_list<float*> outs)
+{
+    const size_t i = (size_t)index;
+    const int64_t n = (int64_t)b->w[i] * b->h[i];
+    Staging dev(b->staging, sizeof(float) * (size_t)n * outs.size());
+    dispatch_batch_storage(b->storage, [&]<class St>() {
+        dim3 g((unsigned)((b->w[i] + 255) / 256), (unsigned)b->h[i]);
+        hipLaunchKernelGGL((k_moments<St, float>), g, dim3(256), 0, b->stream,
+                           (const typename St::S*)lattice_buf(b, index), b->w[i], b->h[i], b->pitch[i], b->plane[i],
+                           batch_consts<typename St::T>(b, index), mask, (float*)dev.get());
+    });
+    CS_HIP(hipGetLastError());
+    const float* src = (const float*)dev.get();
+    for (float* out : outs) {
+        CS_HIP(hipMemcpyAsync(out, src, sizeof(float) * (size_t)n, hipMemcpyDeviceToHost, b->stream));
+        src += n;
+    }
+    CS_HIP(hipStreamSynchronize(b->stream));
+}
+
 extern "C" int cs_batch_velocity(cs_batch* b, int index, float* ux, float* uy)
 {
     return guarded([&] {
         check_batch(b, index);
         CS_REQUIRE(ux && uy, CS_ERR_ARG, "null output");
-        const size_t i = (size_t)index;
-        const int64_t n = (int64_t)b->w[i] * b->h[i];
-        double* dev = nullptr;
-        CS_HIP(hipMalloc(&dev, sizeof(double) * 2 * (size_t)n));
-        dispatch_batch_storage(b->storage, [&]<class St>() {
-            dim3 g((unsigned)((b->w[i] + 255) / 256), (unsigned)b->h[i]);
-            hipLaunchKernelGGL((k_moments<St>), g, dim3(256), 0, b->stream,
-                               (const typename St::S*)lattice_buf(b, index), b->w[i], b->h[i], b->pitch[i],
-                               b->plane[i], batch_consts<typename St::T>(b, index), (unsigned)(M_UX | M_UY), dev);
-        });
-        std::vector<double> host((size_t)(2 * n));
-        hipError_t e = hipGetLastError();
-        hipError_t e1 = hipMemcpyAsync(host.data(), dev, sizeof(double) * 2 * (size_t)n, hipMemcpyDeviceToHost,
-                                       b->stream);
-        hipError_t e2 = hipStreamSynchronize(b->stream);
-        (void)hipFree(dev);
-        CS_HIP(e);
-        CS_HIP(e1);
-        CS_HIP(e2);
-        for (int64_t d = 0; d < n; ++d) {
-            ux[d] = (float)host[(size_t)d];
-            uy[d] = (float)host[(size_t)(n + d)];
-        }
+        batch_moments(b, index, M_UX | M_UY, {ux, uy});
     });
 }
 
@@ -1389,30 +1390,6 @@ extern "C" int cs_batch_moments(cs_batch* b, int index, float* rho, float* ux, f
     return guarded([&] {
         check_batch(b, index);
         CS_REQUIRE(rho && ux && uy, CS_ERR_ARG, "null output");
-        const size_t i = (size_t)index;
-        const int64_t n = (int64_t)b->w[i] * b->h[i];
-        double* dev = nullptr;
-        CS_HIP(hipMalloc(&dev, sizeof(double) * 3 * (size_t)n));
-        dispatch_batch_storage(b->storage, [&]<class St>() {
-            dim3 g((unsigned)((b->w[i] + 255) / 256), (unsigned)b->h[i]);
-            hipLaunchKernelGGL((k_moments<St>), g, dim3(256), 0, b->stream,
-                               (const typename St::S*)lattice_buf(b, index), b->w[i], b->h[i], b->pitch[i],
-                               b->plane[i], batch_consts<typename St::T>(b, index), (unsigned)(M_RHO | M_UX | M_UY),
-                               dev);
-        });
-        std::vector<double> host((size_t)(3 * n));
-        hipError_t e = hipGetLastError();
-        hipError_t e1 = hipMemcpyAsync(host.data(), dev, sizeof(double) * 3 * (size_t)n, hipMemcpyDeviceToHost,
-                                       b->stream);
-        hipError_t e2 = hipStreamSynchronize(b->stream);
-        (void)hipFree(dev);
-        CS_HIP(e);
-        CS_HIP(e1);
-        CS_HIP(e2);
-        for (int64_t d = 0; d < n; ++d) {
-            rho[d] = (float)host[(size_t)d];
-            ux[d] = (float)host[(size_t)(n + d)];
-            uy[d] = (float)host[(size_t)(2 * n + d)];
-        }
+        batch_moments(b, index, M_RHO | M_UX | M_UY, {rho, ux, uy});
     });
 }

@@ -113,6 +113,45 @@ inline bool is_solid_flag(int t) { return t == CS_WALL || t == CS_LID; }
 
 size_t storage_bytes(int storage);
 
+// Device staging of a call's result planes.  A handle keeps one of up to
+// STAGING_KEEP bytes from call to call (hipMalloc and hipFree of a 2 MB
+// buffer take about as long as copying it to the host); larger requests are
+// allocated for the call.  Every user synchronises its stream before it returns.
+constexpr size_t STAGING_KEEP = (size_t)64 << 20;
+struct KeptStaging {
+    void* p = nullptr;
+    size_t bytes = 0;
+};
+class Staging {
+public:
+    Staging(KeptStaging& kept, size_t bytes)
+    {
+        if (bytes > STAGING_KEEP) {
+            CS_HIP(hipMalloc(&own_, bytes));
+            p_ = own_;
+            return;
+        }
+        if (bytes > kept.bytes) {
+            if (kept.p) (void)hipFree(kept.p);
+            kept = KeptStaging{};
+            CS_HIP(hipMalloc(&kept.p, bytes));
+            kept.bytes = bytes;
+        }
+        p_ = kept.p;
+    }
+    ~Staging()
+    {
+        if (own_) (void)hipFree(own_);
+    }
+    Staging(const Staging&) = delete;
+    Staging& operator=(const Staging&) = delete;
+    void* get() const { return p_; }
+
+private:
+    void* p_ = nullptr;
+    void* own_ = nullptr;
+};
+
 }  // namespace cs
 
 struct cs_lattice;
@@ -174,6 +213,7 @@ struct cs_lattice {
     int* iscratch = nullptr;
     double time = 0.0;
     uint64_t steps = 0;         // fused steps taken (keys the stochastic rounding)
+    cs::KeptStaging staging;    // result planes of the moment calls
     void* render_buf = nullptr; // render pass scratch (fields, partials, RGB)
     // Launch-bound lattices replay captured runs of fused steps: one graph per
     // starting buffer parity, valid for the parameters, geometry and launch

@@ -671,29 +671,21 @@ static void init_noalloc_scratch(int device)
 }
 
 // Runs k_moments and copies the requested planes (in mask bit order) to host.
-static void moments_to_host(cs_lattice* l, unsigned mask, double* host)
+template <class Out>
+static void moments_to_host(cs_lattice* l, unsigned mask, Out* const* outs)
 {
     const int nplanes = __builtin_popcount(mask);
     const int64_t n = (int64_t)l->w * l->h;
-    DevBuf out(sizeof(double) * n * nplanes);
+    Staging dev(l->staging, sizeof(Out) * n * nplanes);
     dispatch_storage(l->storage, [&]<class St>() {
-        hipLaunchKernelGGL((k_moments<St>), cell_grid(l), dim3(256), 0, l->stream,
+        hipLaunchKernelGGL((k_moments<St, Out>), cell_grid(l), dim3(256), 0, l->stream,
                            (const typename St::S*)l->buf[l->cur], l->w, l->h, l->pitch, l->plane, consts_of<St>(l),
-                           mask, (double*)out.p);
+                           mask, (Out*)dev.get());
     });
     CS_HIP(hipGetLastError());
-    CS_HIP(hipMemcpyAsync(host, out.p, sizeof(double) * n * nplanes, hipMemcpyDeviceToHost, l->stream));
-    CS_HIP(hipStreamSynchronize(l->stream));
-}
-
-static void moments_f32(cs_lattice* l, unsigned mask, float* const* outs)
-{
-    const int nplanes = __builtin_popcount(mask);
-    const int64_t n = (int64_t)l->w * l->h;
-    std::vector<double> tmp((size_t)n * nplanes);
-    moments_to_host(l, mask, tmp.data());
     for (int j = 0; j < nplanes; ++j)
-        for (int64_t d = 0; d < n; ++d) outs[j][d] = (float)tmp[(size_t)j * n + d];
+        CS_HIP(hipMemcpyAsync(outs[j], (Out*)dev.get() + j * n, sizeof(Out) * n, hipMemcpyDeviceToHost, l->stream));
+    CS_HIP(hipStreamSynchronize(l->stream));
 }
 
 static void reduce(cs_lattice* l, int nv, double* out_host)
@@ -842,7 +834,7 @@ extern "C" int cs_lattice_destroy(cs_lattice* l)
         if (!l) return;
         if (l->stream) (void)hipStreamSynchronize(l->stream);
         for (void* p : {l->buf[0], l->buf[1], (void*)l->flags, (void*)l->node, (void*)l->snap, (void*)l->partials,
-                        (void*)l->dscratch, (void*)l->iscratch, l->render_buf})
+                        (void*)l->dscratch, (void*)l->iscratch, l->render_buf, l->staging.p})
             if (p) (void)hipFree(p);
         clear_step_graphs(l);
         if (l->ev0) (void)hipEventDestroy(l->ev0);
@@ -1238,7 +1230,7 @@ extern "C" int cs_lattice_density(cs_lattice* l, float* rho)
         check_lat(l);
         CS_REQUIRE(rho, CS_ERR_ARG, "null output");
         float* o[] = {rho};
-        moments_f32(l, M_RHO, o);
+        moments_to_host(l, M_RHO, o);
     });
 }
 
@@ -1248,7 +1240,7 @@ extern "C" int cs_lattice_momentum_density(cs_lattice* l, float* mx, float* my)
         check_lat(l);
         CS_REQUIRE(mx && my, CS_ERR_ARG, "null output");
         float* o[] = {mx, my};
-        moments_f32(l, M_MX | M_MY, o);
+        moments_to_host(l, M_MX | M_MY, o);
     });
 }
 
@@ -1258,7 +1250,7 @@ extern "C" int cs_lattice_velocity(cs_lattice* l, float* ux, float* uy)
         check_lat(l);
         CS_REQUIRE(ux && uy, CS_ERR_ARG, "null output");
         float* o[] = {ux, uy};
-        moments_f32(l, M_UX | M_UY, o);
+        moments_to_host(l, M_UX | M_UY, o);
     });
 }
 
@@ -1268,7 +1260,7 @@ extern "C" int cs_lattice_speed(cs_lattice* l, float* speed)
         check_lat(l);
         CS_REQUIRE(speed, CS_ERR_ARG, "null output");
         float* o[] = {speed};
-        moments_f32(l, M_SPEED, o);
+        moments_to_host(l, M_SPEED, o);
     });
 }
 
@@ -1278,7 +1270,7 @@ extern "C" int cs_lattice_pressure(cs_lattice* l, float* p)
         check_lat(l);
         CS_REQUIRE(p, CS_ERR_ARG, "null output");
         float* o[] = {p};
-        moments_f32(l, M_P, o);
+        moments_to_host(l, M_P, o);
     });
 }
 
@@ -1338,12 +1330,13 @@ extern "C" int cs_lattice_moments_f64(cs_lattice* l, double* rho, double* ux, do
 {
     return guarded([&] {
         check_lat(l);
-        const int64_t n = (int64_t)l->w * l->h;
-        std::vector<double> tmp((size_t)(3 * n));
-        moments_to_host(l, M_RHO | M_UX | M_UY, tmp.data());
-        if (rho) std::memcpy(rho, tmp.data(), sizeof(double) * n);
-        if (ux) std::memcpy(ux, tmp.data() + n, sizeof(double) * n);
-        if (uy) std::memcpy(uy, tmp.data() + 2 * n, sizeof(double) * n);
+        const unsigned mask = (rho ? M_RHO : 0u) | (ux ? M_UX : 0u) | (uy ? M_UY : 0u);
+        double* o[3];
+        int k = 0;
+        for (double* p : {rho, ux, uy})
+            if (p) o[k++] = p;
+        if (mask) moments_to_host(l, mask, o);
+        else CS_HIP(hipStreamSynchronize(l->stream));
     });
 }
 

@@ -234,10 +234,11 @@ enum : unsigned {
     M_RHO = 1u, M_MX = 2u, M_MY = 4u, M_UX = 8u, M_UY = 16u, M_SPEED = 32u, M_P = 64u
 };
 
-// Moments of the stored populations into dense double planes.
-template <class St>
+// Moments of the stored populations into dense planes of Out: double, or float
+// for the f32 entry points (the conversion a host loop would make).
+template <class St, class Out = double>
 __global__ void k_moments(const typename St::S* __restrict__ f, int w, int h, int pitch, int64_t P,
-                          Consts<typename St::T> k, unsigned mask, double* __restrict__ out)
+                          Consts<typename St::T> k, unsigned mask, Out* __restrict__ out)
 {
     using T = typename St::T;
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
@@ -249,13 +250,13 @@ __global__ void k_moments(const typename St::S* __restrict__ f, int w, int h, in
     T rho, mx, my, ux, uy;
     moments<St>(k, B, rho, mx, my, ux, uy);
     int slot = 0;
-    if (mask & M_RHO) out[(slot++) * n + d] = (double)rho;
-    if (mask & M_MX) out[(slot++) * n + d] = (double)mx;
-    if (mask & M_MY) out[(slot++) * n + d] = (double)my;
-    if (mask & M_UX) out[(slot++) * n + d] = (double)ux;
-    if (mask & M_UY) out[(slot++) * n + d] = (double)uy;
-    if (mask & M_SPEED) out[(slot++) * n + d] = (double)sqrt(ux * ux + uy * uy);  // lbm.rs:153
-    if (mask & M_P) out[(slot++) * n + d] = (double)(rho * k.cs2);                // lbm.rs:786
+    if (mask & M_RHO) out[(slot++) * n + d] = (Out)rho;
+    if (mask & M_MX) out[(slot++) * n + d] = (Out)mx;
+    if (mask & M_MY) out[(slot++) * n + d] = (Out)my;
+    if (mask & M_UX) out[(slot++) * n + d] = (Out)ux;
+    if (mask & M_UY) out[(slot++) * n + d] = (Out)uy;
+    if (mask & M_SPEED) out[(slot++) * n + d] = (Out)sqrt(ux * ux + uy * uy);  // lbm.rs:153
+    if (mask & M_P) out[(slot++) * n + d] = (Out)(rho * k.cs2);                // lbm.rs:786
 }
 
 
