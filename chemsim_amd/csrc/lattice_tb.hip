@@ -8,8 +8,8 @@
 // microseconds per step: one-step vector kernel 203; K = 2 197, K = 4 137,
 // K = 6 125, K = 8 116 -- beyond 8 the halo's recomputation outgrows the
 // saved traffic; with the region in registers K = 6 measured slower than 8
-// too).  Large lattices without half-way walls take the streaming kernel
-// (lattice_ts.hip).  Otherwise lattices of more than TB_SMALL_MAX_REGIONS 32 x 32 regions (about
+// too).  Large lattices take the streaming kernel (lattice_ts.hip).
+// Otherwise lattices of more than TB_SMALL_MAX_REGIONS 32 x 32 regions (about
 // 512^2) take 64 x 64 regions: k_step_tbr (the region in registers, 73 us
 // per step at 4096^2) without geometry and in the reference boundary mode,
 // k_step_tb (the region in LDS) in the half-way mode, whose link and Zou-He

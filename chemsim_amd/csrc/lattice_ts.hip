@@ -8,14 +8,18 @@
 // shares are known before the launch, so the choice compares them: computed
 // cells per kept cell, the streaming kernel's times 1.12 (what its instruction
 // mix costs more per computed cell; the ratio of measured times to computed
-// cells at 1536^2 .. 8192^2 is 1.07 .. 1.14).  FP32 Taylor-Green, GLUPS,
+// cells at 1536^2 .. 8192^2 is 1.07 .. 1.14; with half-way walls, whose region
+// kernel keeps its cells in LDS, 0.96 .. 1).  FP32 Taylor-Green, GLUPS,
 // streaming / regions in registers: 1024^2 110 / 174, 1536^2 187 / 218,
-// 2048^2 198 / 194, 3072^2 263 / 228, 4096^2 306 / 242, 8192^2 350 / 254.
+// 2048^2 198 / 194, 3072^2 263 / 228, 4096^2 306 / 242, 8192^2 350 / 254;
+// half-way cavity, streaming / regions in LDS: 1536^2 118 / 122, 2001 x 1499
+// 139 / 132, 2048^2 160 / 141, 4096^2 243 / 161, 8192^2 288 / 166; channel with
+// obstacles 2048^2 126 / 108, 4096^2 192 / 118.
 //
 // FP64 has no region kernels (a region would not fit), and its one-step kernel
 // is bound by HBM at 144 bytes per cell update: GLUPS, streaming / one-step,
 // 512^2 50 / 35, 1024^2 92 / 39, 2048^2 126 / 40, 4096^2 162 / 43, half-way
-// cavity 2048^2 82 / 38.  Lattices of 2^20 cells on take it; below that
+// cavity 2048^2 101 / 38.  Lattices of 2^20 cells on take it; below that
 // cs_lattice_temporal_steps goes on reporting one step per launch.  KBC keeps
 // the one-step kernel: its 19 divisions per cell already take as long as the
 // memory, and the strips' recomputation would add to them.
@@ -28,7 +32,8 @@
 //   bf16 stochastic 114 / 111, 130 / 121, 170 / 140, 191 / 150
 //   f16 stochastic 97 / 111, 117 / 118, 150 / 140, 161 / 150
 // so f16 with stochastic rounding takes it only where the fill is small.
-// Half-way walls keep the one-step kernel (f16 cavity 4096^2 103 / 115).
+// Half-way cavity 2048^2 and 4096^2: f16 148 / 99, 224 / 121 to nearest, 101 /
+// 95, 141 / 116 stochastic; bf16 111 / 94, 164 / 115 and 98 / 95, 138 / 118.
 #include "lattice_ts.hpp"
 #include "lbm_tb.hpp"
 
@@ -59,7 +64,8 @@ void ts_coll(cs_lattice* l, int k)
 template <class St, int EDGE>
 void ts_mode(cs_lattice* l, int k)
 {
-    if (l->has_flags) ts_coll<St, EDGE, MODE_REF>(l, k);
+    if (l->has_flags && l->params.boundary == CS_BB_HALFWAY) ts_coll<St, EDGE, MODE_HALF>(l, k);
+    else if (l->has_flags) ts_coll<St, EDGE, MODE_REF>(l, k);
     else ts_coll<St, EDGE, MODE_FLUID>(l, k);
 }
 
@@ -80,20 +86,20 @@ bool ts_takes(const cs_lattice* l)
     if (l->params.collision == CS_COLL_KBC) return false;
     if (l->h < 2 * K) return false;  // the kernel wraps a row index once
     if (l->storage == CS_F64) return (int64_t)l->w * l->h >= (int64_t)1 << 20;
-    if (l->has_flags && l->params.boundary == CS_BB_HALFWAY) return false;
+    const bool half = l->has_flags && l->params.boundary == CS_BB_HALFWAY;
     const TsSplit s = ts_split(l, V, K);
     // both waves of (nearly) every SIMD, or the region kernels' many small blocks win
-    if ((int64_t)s.strips * s.chunks < 6 * (int64_t)l->ctx->prop.multiProcessorCount) return false;
+    if (s.waves() < 6 * (int64_t)l->ctx->prop.multiProcessorCount) return false;
     const double rows = (double)l->h / s.chunks;
     const double stream = (double)s.strips * 64 * V * (rows + K - 1) / ((double)l->w * rows);
     if (storage_bytes(l->storage) == 2) {
         const bool sr = l->params.rounding == CS_ROUND_STOCHASTIC;
-        return stream < (!sr ? 2.2 : l->storage == CS_BF16DEV ? 1.9 : 1.45);
+        return stream < (half ? 1.65 : !sr ? 2.2 : l->storage == CS_BF16DEV ? 1.9 : 1.45);
     }
     constexpr int IN = TB_EDGE - 2 * K;
     const double regions = (double)((l->w + IN - 1) / IN) * ((l->h + IN - 1) / IN) * TB_EDGE * TB_EDGE /
                            ((double)l->w * l->h);
-    return 1.12 * stream < regions;
+    return (half ? 1.0 : 1.12) * stream < regions;
 }
 
 void launch_ts(cs_lattice* l, int k)

@@ -16,17 +16,28 @@ template <class T>
 constexpr int ts_cells() { return sizeof(T) == 8 ? 1 : 2; }
 
 // Waves are independent and all resident at once, two per SIMD; rows are
-// split into as many runs as that allows, of at least 8 rows.
+// split into as many runs as that allows, of at least 8 rows.  Where the
+// lattice's own edge is a wall (half-way mode, zero edge), every row of the
+// first and the last strip takes the geometry pulls and the edge masks, so
+// these strips get more and shorter runs.
 struct TsSplit {
-    int strips, chunks;
+    int strips, chunks, edge_chunks;
+    int64_t waves() const { return (int64_t)std::max(0, strips - 2) * chunks + (int64_t)std::min(strips, 2) * edge_chunks; }
 };
 inline TsSplit ts_split(const cs_lattice* l, int v, int k)
 {
     const int in = 64 * v - 2 * k;
     TsSplit s;
     s.strips = (l->w + in - 1) / in;
-    const int waves = 2 * 4 * std::max(1, l->ctx->prop.multiProcessorCount);
-    s.chunks = std::clamp(waves / s.strips, 1, (l->h + 7) / 8);
+    const int waves = 2 * 4 * std::max(1, l->ctx->prop.multiProcessorCount), most = (l->h + 7) / 8;
+    const bool walls = l->has_flags && l->params.boundary == CS_BB_HALFWAY && l->params.edge == CS_EDGE_ZERO;
+    // an edge strip's time per row in inner strips': cavity and channel 4096^2,
+    // GLUPS with 1, 1.3, 1.6, 2: 206, 226, 243, 242 and 181, 195, 192, 188
+    const double share = walls ? 1.6 : 1.0;
+    const int edges = std::min(s.strips, 2);
+    const double unit = waves / (s.strips - edges + edges * share);
+    s.chunks = std::clamp((int)unit, 1, most);
+    s.edge_chunks = std::clamp((int)(unit * share), 1, most);
     return s;
 }
 
@@ -49,9 +60,10 @@ void ts_launch(cs_lattice* l)
     else A.a.k = l->k32;
     A.strips = sp.strips;
     A.chunks = sp.chunks;
+    A.edge_chunks = sp.edge_chunks;
     if constexpr (SR)
         for (int s = 0; s < K; ++s) A.keys[s] = sr_key(l->params.seed, l->steps + (uint64_t)s);
-    const unsigned blocks = (unsigned)(((int64_t)A.strips * A.chunks + TS_WAVES - 1) / TS_WAVES);
+    const unsigned blocks = (unsigned)((sp.waves() + TS_WAVES - 1) / TS_WAVES);
     hipLaunchKernelGGL((k_step_ts<St, EDGE, MODE, K, COLL, V, SR>), dim3(blocks), dim3(TS_THREADS), 0, l->stream, A);
     l->cur ^= 1;
     l->steps += K;

@@ -50,7 +50,8 @@ constexpr int TS_RING = 16;                // rows of node words kept (>= K + 1,
 template <class T, int K>
 struct TsArgs {
     StepArgs<T> a;
-    int strips, chunks;   // waves: strips x chunks
+    int strips, chunks;   // waves: chunks per inner strip,
+    int edge_chunks;      // and per first and last strip
     uint32_t keys[K];     // stochastic rounding keys of the K steps
 };
 
@@ -106,6 +107,30 @@ __device__ __forceinline__ void ts_round(float (&x)[9], uint32_t cell_key)
     }
 }
 
+// All ones where bit `bit` of w is set.  Kept as a mask in a vector register:
+// as a condition it would be a compare into scalar registers and, after two
+// wait states, a select per value.
+__device__ __forceinline__ uint32_t ts_mask(uint32_t w, int bit)
+{
+    uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)w, (unsigned)bit, 1u);
+    asm volatile("" : "+v"(m));
+    return m;
+}
+// m ? a : b
+template <class T>
+__device__ __forceinline__ T ts_select(uint32_t m, T a, T b)
+{
+    if constexpr (sizeof(T) == 8) {
+        const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+        const uint32_t lo = (m & (uint32_t)x) | (~m & (uint32_t)y);
+        const uint32_t hi = (m & (uint32_t)(x >> 32)) | (~m & (uint32_t)(y >> 32));
+        return __builtin_bit_cast(T, ((uint64_t)hi << 32) | lo);
+    } else {
+        const uint32_t x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
+        return __builtin_bit_cast(T, (m & x) | (~m & y));
+    }
+}
+
 // Per-wave LDS of the geometry modes.
 template <class T, int MODE, int K, int V>
 struct TsLds {
@@ -127,7 +152,7 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
     using S = typename St::S;
     using T = typename St::T;
     constexpr bool HALF = MODE == MODE_HALF;
-    constexpr int UNROLL = HALF ? 1 : 2;
+    constexpr int UNROLL = HALF ? 1 : 2;  // the half-way mode's loop is too long to repeat
     const StepArgs<T>& a = A.a;
     const int lane = (int)(threadIdx.x & 63);
     const int lprev = ((lane - 1) & 63) * 4, lnext = ((lane + 1) & 63) * 4;
@@ -150,6 +175,9 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
         }
         col[j] = (uint32_t)c;
     }
+    uint32_t inside[V];  // cin as a vector mask
+#pragma unroll
+    for (int j = 0; j < V; ++j) inside[j] = ts_mask(cin[j], 0);
     const bool edge_strip = EDGE == CS_EDGE_ZERO && (c0 < 0 || c0 + 64 * V > a.w);  // uniform over the wave
     const bool vec_out = V == 1 || c0 + 64 * V - K <= a.w || a.w % V == 0;  // the lane's cells stored as one vector
     const auto outside = [&](int i) -> T { return St::DEV ? -a.k.base(i) : T(0); };
@@ -191,9 +219,10 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
         bool in;
         wrap_row(r, in);
 #pragma unroll
-        for (int j = 0; j < V; ++j) {
-            x[j] = St::wid(P[i][j]);
-            if (EDGE == CS_EDGE_ZERO) x[j] = in && cin[j] ? x[j] : outside(i);
+        for (int j = 0; j < V; ++j) x[j] = St::wid(P[i][j]);
+        if (EDGE == CS_EDGE_ZERO && (edge_strip || !in)) {  // uniform over the wave
+#pragma unroll
+            for (int j = 0; j < V; ++j) x[j] = ts_select(in ? inside[j] : 0u, x[j], outside(i));
         }
     };
 
@@ -207,7 +236,8 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
 
     const int iters = (rb - ra) + 2 * (K - 1);
     int r1 = ra - (K - 1);  // level 1's row
-    uint32_t special = 0;   // bit s - 1: level s's row needs the geometry pulls
+    // bit s - 1: level s's row needs the geometry pulls; has a lid link; has an inlet or outlet cell
+    uint32_t special = 0, lid_rows = 0, io_rows = 0;
     if constexpr (HALF) {
         // populations 3, 6, 7 of the row above the first, and 1, 5, 8 of the first row itself
         load3(r1 - 1, DN);
@@ -234,7 +264,7 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
             take(DN[q], HALF ? r1 : r1 - 1, N[DN[q]]);
         }
         if constexpr (MODE != MODE_FLUID) {
-            bool in, need = false;
+            bool in, need = false, lid = false, io = false;
             wrap_row(r1, in);
 #pragma unroll
             for (int j = 0; j < V; ++j) {
@@ -242,9 +272,15 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
                 const int type = (int)(w >> NODE_TYPE_SHIFT);
                 const bool solid = type == CS_WALL || type == CS_LID;
                 need = need || solid || (HALF && ((w & 0x1FEu) != 0 || type != CS_FLUID));
+                lid = lid || (w & 0x3FC00u) != 0;
+                io = io || type == CS_INLET || type == CS_OUTLET;
                 lds->ring[r1 & (TS_RING - 1)][lane * V + j] = w;
             }
             special = (special << 1) | (__any(need) ? 1u : 0u);
+            if (HALF) {
+                lid_rows = (lid_rows << 1) | (__any(lid) ? 1u : 0u);
+                io_rows = (io_rows << 1) | (__any(io) ? 1u : 0u);
+            }
         }
         load_row(r1 + 1);
 
@@ -328,23 +364,29 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
                     const int type = (int)(info[j] >> NODE_TYPE_SHIFT);
                     const bool solid = type == CS_WALL || type == CS_LID;
                     if constexpr (MODE == MODE_REF) {
+                        const uint32_t swap = ts_mask(solid, 0);
 #pragma unroll
                         for (int i = 1; i < 9; ++i)
                             if (i < OPP[i]) {
                                 const T x = C[j][i], y = C[j][OPP[i]];
-                                C[j][i] = solid ? y : x;
-                                C[j][OPP[i]] = solid ? x : y;
+                                C[j][i] = ts_select(swap, y, x);
+                                C[j][OPP[i]] = ts_select(swap, x, y);
                             }
                     } else if constexpr (HALF) {
                         const T own[9] = {um[0][j], u1[0][j], um[1][j], dc[0][j], um[2][j],
                                           u1[1][j], dc[1][j], dc[2][j], u1[2][j]};
+                        const uint32_t links = solid ? 0u : info[j];
+                        if ((lid_rows >> (s - 1)) & 1u) {  // uniform
 #pragma unroll
-                        for (int i = 1; i < 9; ++i)
-                            if (!solid && ((info[j] >> i) & 1u)) {
-                                T v = own[OPP[i]];
-                                if ((info[j] >> (9 + i)) & 1u) v = v + a.k.lid(i);
-                                C[j][i] = v;
+                            for (int i = 1; i < 9; ++i) {
+                                const T v = own[OPP[i]];
+                                C[j][i] = ts_select(ts_mask(links, i), ts_select(ts_mask(links, 9 + i), v + a.k.lid(i), v), C[j][i]);
                             }
+                        } else {
+#pragma unroll
+                            for (int i = 1; i < 9; ++i) C[j][i] = ts_select(ts_mask(links, i), own[OPP[i]], C[j][i]);
+                        }
+                        if ((io_rows >> (s - 1)) & 1u) {  // uniform
                         if constexpr (St::DEV) {
                             if (type == CS_INLET) zou_he_inlet_dev<T>(C[j], a.k.rho0, a.k.in_ux, a.k.in_uy);
                             else if (type == CS_OUTLET) zou_he_outlet_dev<T>(C[j], a.k.rho0, a.k.out_rho);
@@ -352,8 +394,14 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
                             if (type == CS_INLET) zou_he_inlet<T>(C[j], a.k.in_ux, a.k.in_uy);
                             else if (type == CS_OUTLET) zou_he_outlet<T>(C[j], a.k.out_rho);
                         }
+                        }
                     }
                 }
+            }
+            if (EDGE == CS_EDGE_ZERO && edge_strip) {
+                // cells outside keep the outside value (below); a rho of 1 keeps them off the reciprocal's branch
+#pragma unroll
+                for (int j = 0; j < V; ++j) C[j][0] = ts_select(inside[j], C[j][0], T(1));
             }
             if constexpr (V == 1) {
                 collide_cell<St, COLL>(a.k, C[0]);
@@ -383,11 +431,11 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
 #pragma unroll
                     for (int j = 0; j < V; ++j) {
                         const int type = (int)(info[j] >> NODE_TYPE_SHIFT);
-                        const bool solid = type == CS_WALL || type == CS_LID;  // carried unchanged
+                        const uint32_t solid = ts_mask(type == CS_WALL || type == CS_LID, 0);  // carried unchanged
                         const T own[9] = {um[0][j], u1[0][j], um[1][j], dc[0][j], um[2][j],
                                           u1[1][j], dc[1][j], dc[2][j], u1[2][j]};
 #pragma unroll
-                        for (int i = 0; i < 9; ++i) C[j][i] = solid ? own[i] : C[j][i];
+                        for (int i = 0; i < 9; ++i) C[j][i] = ts_select(solid, own[i], C[j][i]);
                     }
                 }
             }
@@ -397,7 +445,7 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
 #pragma unroll
                     for (int j = 0; j < V; ++j)
 #pragma unroll
-                        for (int i = 0; i < 9; ++i) C[j][i] = rin && cin[j] ? C[j][i] : outside(i);
+                        for (int i = 0; i < 9; ++i) C[j][i] = ts_select(rin ? inside[j] : 0u, C[j][i], outside(i));
                 }
             }
 #pragma unroll
@@ -459,9 +507,21 @@ __global__ __launch_bounds__(TS_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
     __shared__ Lds lds[MODE == MODE_FLUID ? 1 : TS_WAVES];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int id = xcd_tile(blockIdx.x, gridDim.x) * TS_WAVES + wave;
-    if (id >= A.strips * A.chunks) return;
-    const int chunk = id / A.strips, strip = id - chunk * A.strips;
-    const int ra = (int)((int64_t)A.a.h * chunk / A.chunks), rb = (int)((int64_t)A.a.h * (chunk + 1) / A.chunks);
+    // the first and the last strip's chunks come first
+    const int edges = A.strips > 1 ? 2 : 1, outer = edges * A.edge_chunks;
+    int strip, chunk, chunks;
+    if (id < outer) {
+        strip = id < A.edge_chunks ? 0 : A.strips - 1;
+        chunk = id < A.edge_chunks ? id : id - A.edge_chunks;
+        chunks = A.edge_chunks;
+    } else {
+        const int inner = A.strips - edges, k = id - outer;
+        if (inner <= 0 || k >= inner * A.chunks) return;
+        chunk = k / inner;
+        strip = 1 + k - chunk * inner;
+        chunks = A.chunks;
+    }
+    const int ra = (int)((int64_t)A.a.h * chunk / chunks), rb = (int)((int64_t)A.a.h * (chunk + 1) / chunks);
     ts_strip<St, EDGE, MODE, K, COLL, V, SR>(A, strip * (64 * V - 2 * K) - K, ra, rb,
                                              &lds[MODE == MODE_FLUID ? 0 : wave]);
 }

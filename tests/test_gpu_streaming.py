@@ -36,6 +36,40 @@ def test_bgk_matches_oracle(ctx, shape, masked, edge):
         np.testing.assert_array_equal(lat.download(), O.run(op, f, 21, flags))
 
 
+@pytest.mark.parametrize("edge", [O.EDGE_ZERO, O.EDGE_PERIODIC])
+@pytest.mark.parametrize("shape", SHAPES, ids=[f"{w}x{h}" for w, h in SHAPES])
+def test_halfway_matches_oracle(ctx, shape, edge):
+    w, h = shape
+    rng = np.random.default_rng(68)
+    f = rand_state(rng, h, w)
+    flags = random_flags(rng, h, w)
+    flags[:, w // 3:] = 0
+    flags[h // 2:] = 0
+    op = O.params(w, h, tau=0.62, edge=edge, boundary=O.BB_HALFWAY, lid=(0.02, -0.03))
+    with Lattice(ctx, w, h, "f32", gpu_params(op), flags) as lat:
+        assert lat.temporal_steps() == 8
+        lat.upload(f)
+        lat.step(13)
+        np.testing.assert_array_equal(lat.download(), O.run(op, f, 13, flags))
+
+
+@pytest.mark.parametrize("storage", ["f32", "f32dev"])
+def test_channel_matches_oracle(ctx, storage):
+    ch = W.Channel(w=3001, h=1802, circles=[(900, 700, 160), (400, 2000, 90)], re=60.0, u_in=0.05)
+    flags = ch.flags()
+    op = O.params(ch.w, ch.h, tau=max(ch.tau, 0.55), boundary=O.BB_HALFWAY, inlet=ch.inlet(), outlet_rho=1.0)
+    rho, ux, uy = W.rest_state(ch.w, ch.h)
+    with Lattice(ctx, ch.w, ch.h, storage, gpu_params(op), flags) as lat:
+        lat.init_equilibrium(rho, ux, uy)
+        lat.step(20)
+        if storage == "f32":
+            f0 = O.equilibrium(op, rho, ux, uy).astype(np.float32)
+            np.testing.assert_array_equal(lat.download(), O.run(op, f0, 20, flags))
+        else:
+            g0 = O.equilibrium_dev(op, rho, ux, uy)
+            np.testing.assert_array_equal(lat.download_raw(), O.run_devf32(op, g0, 20, flags))
+
+
 @pytest.mark.parametrize("coll", ["trt", "regularized"])
 def test_operators_match_oracle(ctx, coll):
     w, h = SHAPES[1]
@@ -134,7 +168,7 @@ def test_f64_channel_matches_one_step(ctx):
 
 
 @pytest.mark.parametrize("edge", [O.EDGE_ZERO, O.EDGE_PERIODIC])
-@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("masked", [None, "reference", "halfway"])
 @pytest.mark.parametrize("rounding", [capi.CS_ROUND_NEAREST, capi.CS_ROUND_STOCHASTIC], ids=["nearest", "stochastic"])
 @pytest.mark.parametrize("storage", ["bf16", "f16"])
 def test_16bit_matches_one_step(ctx, storage, rounding, masked, edge):
@@ -150,7 +184,8 @@ def test_16bit_matches_one_step(ctx, storage, rounding, masked, edge):
     flags = random_flags(rng, h, w) if masked else None
     if masked:
         flags[:, w // 3:] = 0
-    p = Params(tau=0.7, edge=edge, rounding=rounding, seed=9)
+    p = Params(tau=0.7, edge=edge, rounding=rounding, seed=9, lid_uy=0.03,
+               boundary=capi.CS_BB_HALFWAY if masked == "halfway" else capi.CS_BB_REFERENCE)
     out = []
     try:
         for k in (capi.CS_TEMPORAL_AUTO, 0):
