@@ -537,6 +537,30 @@ __device__ __forceinline__ void bgk_collide_dev(const Consts<T>& k, X (&B)[9])
     }
 }
 
+// All ones where bit `bit` of w is set.  Kept as a mask in a vector register:
+// as a condition it would be a compare into scalar registers and, after two
+// wait states, a select per value.
+__device__ __forceinline__ uint32_t lane_mask(uint32_t w, int bit)
+{
+    uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)w, (unsigned)bit, 1u);
+    asm volatile("" : "+v"(m));
+    return m;
+}
+// m ? a : b
+template <class T>
+__device__ __forceinline__ T lane_select(uint32_t m, T a, T b)
+{
+    if constexpr (sizeof(T) == 8) {
+        const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+        const uint32_t lo = (m & (uint32_t)x) | (~m & (uint32_t)y);
+        const uint32_t hi = (m & (uint32_t)(x >> 32)) | (~m & (uint32_t)(y >> 32));
+        return __builtin_bit_cast(T, ((uint64_t)hi << 32) | lo);
+    } else {
+        const uint32_t x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
+        return __builtin_bit_cast(T, (m & x) | (~m & y));
+    }
+}
+
 // Zou-He on deviations: the unknown populations follow the same formulas
 // (opposite directions share w_i); only the density sums carry rho0.
 template <class T>

@@ -107,30 +107,6 @@ __device__ __forceinline__ void ts_round(float (&x)[9], uint32_t cell_key)
     }
 }
 
-// All ones where bit `bit` of w is set.  Kept as a mask in a vector register:
-// as a condition it would be a compare into scalar registers and, after two
-// wait states, a select per value.
-__device__ __forceinline__ uint32_t ts_mask(uint32_t w, int bit)
-{
-    uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)w, (unsigned)bit, 1u);
-    asm volatile("" : "+v"(m));
-    return m;
-}
-// m ? a : b
-template <class T>
-__device__ __forceinline__ T ts_select(uint32_t m, T a, T b)
-{
-    if constexpr (sizeof(T) == 8) {
-        const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
-        const uint32_t lo = (m & (uint32_t)x) | (~m & (uint32_t)y);
-        const uint32_t hi = (m & (uint32_t)(x >> 32)) | (~m & (uint32_t)(y >> 32));
-        return __builtin_bit_cast(T, ((uint64_t)hi << 32) | lo);
-    } else {
-        const uint32_t x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
-        return __builtin_bit_cast(T, (m & x) | (~m & y));
-    }
-}
-
 // Per-wave LDS of the geometry modes.
 template <class T, int MODE, int K, int V>
 struct TsLds {
@@ -177,7 +153,7 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
     }
     uint32_t inside[V];  // cin as a vector mask
 #pragma unroll
-    for (int j = 0; j < V; ++j) inside[j] = ts_mask(cin[j], 0);
+    for (int j = 0; j < V; ++j) inside[j] = lane_mask(cin[j], 0);
     const bool edge_strip = EDGE == CS_EDGE_ZERO && (c0 < 0 || c0 + 64 * V > a.w);  // uniform over the wave
     const bool vec_out = V == 1 || c0 + 64 * V - K <= a.w || a.w % V == 0;  // the lane's cells stored as one vector
     const auto outside = [&](int i) -> T { return St::DEV ? -a.k.base(i) : T(0); };
@@ -222,7 +198,7 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
         for (int j = 0; j < V; ++j) x[j] = St::wid(P[i][j]);
         if (EDGE == CS_EDGE_ZERO && (edge_strip || !in)) {  // uniform over the wave
 #pragma unroll
-            for (int j = 0; j < V; ++j) x[j] = ts_select(in ? inside[j] : 0u, x[j], outside(i));
+            for (int j = 0; j < V; ++j) x[j] = lane_select(in ? inside[j] : 0u, x[j], outside(i));
         }
     };
 
@@ -364,13 +340,13 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
                     const int type = (int)(info[j] >> NODE_TYPE_SHIFT);
                     const bool solid = type == CS_WALL || type == CS_LID;
                     if constexpr (MODE == MODE_REF) {
-                        const uint32_t swap = ts_mask(solid, 0);
+                        const uint32_t swap = lane_mask(solid, 0);
 #pragma unroll
                         for (int i = 1; i < 9; ++i)
                             if (i < OPP[i]) {
                                 const T x = C[j][i], y = C[j][OPP[i]];
-                                C[j][i] = ts_select(swap, y, x);
-                                C[j][OPP[i]] = ts_select(swap, x, y);
+                                C[j][i] = lane_select(swap, y, x);
+                                C[j][OPP[i]] = lane_select(swap, x, y);
                             }
                     } else if constexpr (HALF) {
                         const T own[9] = {um[0][j], u1[0][j], um[1][j], dc[0][j], um[2][j],
@@ -380,11 +356,11 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
 #pragma unroll
                             for (int i = 1; i < 9; ++i) {
                                 const T v = own[OPP[i]];
-                                C[j][i] = ts_select(ts_mask(links, i), ts_select(ts_mask(links, 9 + i), v + a.k.lid(i), v), C[j][i]);
+                                C[j][i] = lane_select(lane_mask(links, i), lane_select(lane_mask(links, 9 + i), v + a.k.lid(i), v), C[j][i]);
                             }
                         } else {
 #pragma unroll
-                            for (int i = 1; i < 9; ++i) C[j][i] = ts_select(ts_mask(links, i), own[OPP[i]], C[j][i]);
+                            for (int i = 1; i < 9; ++i) C[j][i] = lane_select(lane_mask(links, i), own[OPP[i]], C[j][i]);
                         }
                         if ((io_rows >> (s - 1)) & 1u) {  // uniform
                         if constexpr (St::DEV) {
@@ -401,7 +377,7 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
             if (EDGE == CS_EDGE_ZERO && edge_strip) {
                 // cells outside keep the outside value (below); a rho of 1 keeps them off the reciprocal's branch
 #pragma unroll
-                for (int j = 0; j < V; ++j) C[j][0] = ts_select(inside[j], C[j][0], T(1));
+                for (int j = 0; j < V; ++j) C[j][0] = lane_select(inside[j], C[j][0], T(1));
             }
             if constexpr (V == 1) {
                 collide_cell<St, COLL>(a.k, C[0]);
@@ -431,11 +407,11 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
 #pragma unroll
                     for (int j = 0; j < V; ++j) {
                         const int type = (int)(info[j] >> NODE_TYPE_SHIFT);
-                        const uint32_t solid = ts_mask(type == CS_WALL || type == CS_LID, 0);  // carried unchanged
+                        const uint32_t solid = lane_mask(type == CS_WALL || type == CS_LID, 0);  // carried unchanged
                         const T own[9] = {um[0][j], u1[0][j], um[1][j], dc[0][j], um[2][j],
                                           u1[1][j], dc[1][j], dc[2][j], u1[2][j]};
 #pragma unroll
-                        for (int i = 0; i < 9; ++i) C[j][i] = ts_select(solid, own[i], C[j][i]);
+                        for (int i = 0; i < 9; ++i) C[j][i] = lane_select(solid, own[i], C[j][i]);
                     }
                 }
             }
@@ -445,7 +421,7 @@ __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int
 #pragma unroll
                     for (int j = 0; j < V; ++j)
 #pragma unroll
-                        for (int i = 0; i < 9; ++i) C[j][i] = ts_select(rin ? inside[j] : 0u, C[j][i], outside(i));
+                        for (int i = 0; i < 9; ++i) C[j][i] = lane_select(rin ? inside[j] : 0u, C[j][i], outside(i));
                 }
             }
 #pragma unroll
