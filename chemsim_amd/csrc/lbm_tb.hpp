@@ -69,7 +69,10 @@ __device__ __forceinline__ void tb_gather(const typename St::T (&L)[9][RE][RE], 
                                           typename St::T (&B)[9])
 {
     using T = typename St::T;
-    const int type = MODE == MODE_FLUID ? (int)CS_FLUID : (int)(info >> NODE_TYPE_SHIFT);
+    int type = MODE == MODE_FLUID ? (int)CS_FLUID : (int)(info >> NODE_TYPE_SHIFT);
+    // a plain register: compares that select the byte themselves (SDWA) are slow to
+    // issue (recip_newton's comment); channels 2-5% at 64^2 .. 1500^2
+    if (MODE == MODE_HALF) asm volatile("" : "+v"(type));
     const bool solid = type == CS_WALL || type == CS_LID;
 #pragma unroll
     for (int i = 0; i < 9; ++i) B[i] = L[i][rr + CX[i]][(lane - CY[i]) & (RE - 1)];
@@ -208,8 +211,25 @@ __device__ __forceinline__ void tb_region(const StepArgs<typename St::T>& a, int
         for (int j = 0; j < SLOTS; ++j) {
             const int rr = row0 + RSTRIDE * j;
             if (rr >= s && rr < RE - s) {  // uniform over the wave at RE = 64
-                tb_gather<St, MODE, RE>(L, rr, lane, info[j], special[j], linked[j], lid[j], io[j], a.k, B[j]);
-                collide_cell<St, COLL>(a.k, B[j]);
+                uint32_t word = info[j];
+                // keeps the link conditions out of the loop's scalar registers: 32 lane masks
+                // held from step to step spilled 102 of them to vector lanes
+                if (MODE == MODE_HALF && RE == TB_EDGE) asm volatile("" : "+v"(word));
+                tb_gather<St, MODE, RE>(L, rr, lane, word, special[j], linked[j], lid[j], io[j], a.k, B[j]);
+                if constexpr (RE == TB_EDGE_SMALL && MODE == MODE_HALF) {
+                    // recip_newton: cavity 128^2 1.46 -> 1.38 us per step, 512^2 3.64 ->
+                    // 3.51.  Without half-way walls its five more instructions cost more
+                    // than they give (periodic 128^2 1.14 -> 1.25); 64 x 64 regions
+                    // measured the same either way.
+                    Cells<T, 1> X[9];
+#pragma unroll
+                    for (int i = 0; i < 9; ++i) X[i].v[0] = B[j][i];
+                    collide_cell<St, COLL>(a.k, X);
+#pragma unroll
+                    for (int i = 0; i < 9; ++i) B[j][i] = X[i].v[0];
+                } else {
+                    collide_cell<St, COLL>(a.k, B[j]);
+                }
             }
         }
         __syncthreads();  // every read of step s done before any write
