@@ -390,7 +390,7 @@ void gemm(cs_cnn* net, int la, int lb, int epi, const uint16_t* A, int lda, cons
     CS_REQUIRE(K % 8 == 0, CS_ERR_ARG, "gemm K must be a multiple of 8");
     g.k_per_split = ((K + splits - 1) / splits + BK - 1) / BK * BK;  // splits cover [0, K)
     g.split_stride = (int64_t)M * ldc;
-    const int cfg = pick_tile(M, N);
+    const int cfg = la == GATHER && splits == 1 ? pick_gather_tile(M, N) : pick_tile(M, N);
     int bm, bn;
     tile_dims(cfg, bm, bn);
     dim3 grid((unsigned)((M + bm - 1) / bm), (unsigned)((N + bn - 1) / bn), (unsigned)splits);
