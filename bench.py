@@ -70,10 +70,46 @@ def tb_bytes_per_step(w: int, h: int, esize: int = 4, k: int = TB_STEPS, edge: i
     return (regions * edge * edge + w * h) * 9 * esize / k
 
 
-def step_bytes_per_cell(storage: str, n: int, k: int) -> float:
+def ts_split(w: int, h: int, storage: str, k: int = TB_STEPS) -> tuple[int, int, int]:
+    """Columns per strip, strips and runs of rows per strip of the streaming
+    kernel on a lattice without walls (two waves per SIMD of 256 CUs)."""
+    cols = 64 if storage == "f64" else 128
+    strips = -(-w // (cols - 2 * k))
+    return cols, strips, max(1, min(2048 // strips, (h + 7) // 8))
+
+
+def ts_takes(w: int, h: int, storage: str, rounding: str = "sr") -> bool:
+    """Whether a periodic BGK lattice takes the streaming kernel (the rule of
+    chemsim_amd/csrc/lattice_ts.hip)."""
+    if h < 16:
+        return False
+    if storage == "f64":
+        return w * h >= 1 << 20
+    cols, strips, chunks = ts_split(w, h, storage)
+    if strips * chunks < 1536:
+        return False
+    rows = h / chunks
+    stream = strips * cols * (rows + TB_STEPS - 1) / (w * rows)
+    if storage in ("f16", "bf16"):
+        return stream < (2.2 if rounding != "sr" else 1.9 if storage == "bf16" else 1.45)
+    inner = TB_EDGE - 2 * TB_STEPS
+    return 1.12 * stream < -(-w // inner) * -(-h // inner) * TB_EDGE * TB_EDGE / (w * h)
+
+
+def ts_bytes_per_step(w: int, h: int, storage: str, k: int = TB_STEPS) -> float:
+    """Bytes one launch of the streaming kernel must move, per step: every run
+    reads its rows and k more on either side over the strip's columns, every
+    lattice cell is written once."""
+    cols, strips, chunks = ts_split(w, h, storage, k)
+    return (strips * cols * (h + 2 * k * chunks) + w * h) * BYTES_PER_CELL[storage] / 2 / k
+
+
+def step_bytes_per_cell(storage: str, n: int, k: int, rounding: str = "sr") -> float:
     """Algorithmic bytes per cell update of the kernel an n x n lattice takes
     (k: steps per launch, Lattice.temporal_steps(); 1 = a one-step kernel)."""
     if k > 1:
+        if ts_takes(n, n, storage, rounding):
+            return ts_bytes_per_step(n, n, storage, k) / (n * n)
         return tb_bytes_per_step(n, n, k=k) / (n * n)
     return BYTES_PER_CELL[storage]
 
@@ -92,10 +128,23 @@ def run_bytes_per_cell(storage: str, n: int, k: int, steps: int) -> float:
     return total / (n * n * steps)
 
 
-def warm_kernels(ctx, n, storage, tau, u0):
+def launched_bytes_per_cell(storage: str, n: int, k: int, steps: int) -> float:
+    """run_bytes_per_cell with the streaming kernel's bytes where an n x n
+    lattice takes it (a remainder of 4 steps as one 4-step launch for 4- and
+    8-byte storage)."""
+    if k <= 1 or not ts_takes(n, n, storage):
+        return run_bytes_per_cell(storage, n, k, steps)
+    nk, r = divmod(steps, k)
+    n4 = 1 if r >= 4 and BYTES_PER_CELL[storage] > 36 else 0
+    total = nk * k * ts_bytes_per_step(n, n, storage, k) + n4 * 4 * ts_bytes_per_step(n, n, storage, 4) \
+        + (r - 4 * n4) * n * n * BYTES_PER_CELL[storage]
+    return total / (n * n * steps)
+
+
+def warm_kernels(ctx, n, storage, tau, u0, rounding="sr"):
     """One launch of each step kernel a run on this lattice shape uses (the
     8-step, 4-step and one-step launches of 13 steps), on a scratch lattice."""
-    with tgv_lattice(ctx, n, storage, tau, u0) as scratch:
+    with tgv_lattice(ctx, n, storage, tau, u0, rounding) as scratch:
         scratch.step(13)
         scratch.sync()
 
@@ -401,7 +450,7 @@ def main():
     kernel_ms = ms / args.steps
     k_launch = lat.temporal_steps()
     temporal = k_launch > 1
-    bpc = run_bytes_per_cell(storage, n, k_launch, args.steps)
+    bpc = launched_bytes_per_cell(storage, n, k_launch, args.steps)
     achieved = bpc * cells / (kernel_ms * 1e-3) / 1e9
     log(f"[bench] {glups:.2f} GLUPS wall, {kernel_ms * 1e3:.1f} us/step (events), {achieved:.0f} GB/s algorithmic")
     # four more timed regions of the same length, for the spread (value stays the first)
@@ -440,7 +489,7 @@ def main():
                                      "kernel_us": round(ms1 / args.steps * 1e3, 2),
                                      "hbm_frac": hbm_frac(BYTES_PER_CELL[storage], cells, ms1 / args.steps),
                                      "bytes_per_cell": BYTES_PER_CELL[storage]}
-        extras["temporal_blocking"] = {"steps_per_launch": k_launch, "region": [tb_region_edge(n, n)] * 2,
+        extras["temporal_blocking"] = {"steps_per_launch": k_launch, "kernel": "streaming" if ts_takes(n, n, storage) else "regions",
                                        "bytes_per_cell_update": round(bpc, 3),
                                        "speedup_vs_one_step": round(extras["one_step_kernel"]["kernel_us"]
                                                                     / (kernel_ms * 1e3), 3)}
@@ -450,14 +499,17 @@ def main():
         # FP64 oracle run and 16-bit storage on the same workload, same steps
         from chemsim_amd import workloads as W
         lat.close()
+        warm_kernels(ctx, n, "f64", args.tau, args.u0)
         ref = tgv_lattice(ctx, n, "f64", args.tau, args.u0)
+        k64 = ref.temporal_steps()
         m0 = ref.sums_f64()[0]
         w64, ms64 = time_steps(ref, args.steps)
         r64, x64, y64 = ref.moments_f64()
         m1 = ref.sums_f64()[0]
         ref.close()
         extras["f64"] = {"GLUPS": round(cells * args.steps / w64 / 1e9, 3),
-                         "hbm_frac": hbm_frac(144, cells, ms64 / args.steps),
+                         "hbm_frac": hbm_frac(step_bytes_per_cell("f64", n, k64), cells, ms64 / args.steps),
+                         "steps_per_launch": k64,
                          "mass_drift_rel": abs(m1 - m0) / m0}
         amp = W.taylor_green_decay(n, args.tau, args.steps)
         rho0, ux0, uy0 = W.taylor_green(n, args.u0)
@@ -468,6 +520,7 @@ def main():
         rden = np.sqrt(((r64 - 1.0) ** 2).sum())
         for st, rnd in (("f32", "rn"), ("f32dev", "rn"), ("bf16", "sr"), ("f16", "sr"), ("bf16", "rn"),
                         ("f16", "rn")):
+            warm_kernels(ctx, n, st, args.tau, args.u0, rnd)
             l2 = tgv_lattice(ctx, n, st, args.tau, args.u0, rnd)
             k2 = l2.temporal_steps()
             m0 = l2.sums_f64()[0]
@@ -477,7 +530,7 @@ def main():
             l2.close()
             key = st if st in ("f32", "f32dev") else f"{st}_{rnd}"
             extras[key] = {"GLUPS": round(cells * args.steps / w2 / 1e9, 3),
-                          "hbm_frac": hbm_frac(step_bytes_per_cell(st, n, k2), cells, ms2 / args.steps),
+                          "hbm_frac": hbm_frac(step_bytes_per_cell(st, n, k2, rnd), cells, ms2 / args.steps),
                           "steps_per_launch": k2,
                           "u_rel_L2_vs_f64": float(np.sqrt(((x - x64) ** 2 + (y - y64) ** 2).sum()) / den),
                           "rho_dev_rel_L2_vs_f64": float(np.sqrt(((r - r64) ** 2).sum()) / rden),

@@ -9,7 +9,7 @@
 // has just computed, the others are kept in registers -- only the populations
 // that are still to be pulled: 0, 2, 4 of row r' and 3, 6, 7 of rows r' and
 // r' - 1, nine values per cell and level.  Neighbouring columns come from the
-// lane itself or by a DPP wave shift.  No LDS, no barrier and no
+// lane itself or from the next lane (ts_lane).  No barrier and no
 // communication between waves; the per-cell arithmetic and pull order are the
 // one-step kernels', so K steps equal K launches of k_step bit for bit.
 //
