@@ -1209,12 +1209,7 @@ static void batch_moments(cs_batch* b, int index, unsigned mask, std::initialize
                            batch_consts<typename St::T>(b, index), mask, (float*)dev.get());
     });
     CS_HIP(hipGetLastError());
-    const float* src = (const float*)dev.get();
-    for (float* out : outs) {
-        CS_HIP(hipMemcpyAsync(out, src, sizeof(float) * (size_t)n, hipMemcpyDeviceToHost, b->stream));
-        src += n;
-    }
-    CS_HIP(hipStreamSynchronize(b->stream));
+    planes_to_host((const float*)dev.get(), n, outs.begin(), (int)outs.size(), b->stream);
 }
 
 extern "C" int cs_batch_velocity(cs_batch* b, int index, float* ux, float* uy)

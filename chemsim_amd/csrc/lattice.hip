@@ -683,9 +683,7 @@ static void moments_to_host(cs_lattice* l, unsigned mask, Out* const* outs)
                            mask, (Out*)dev.get());
     });
     CS_HIP(hipGetLastError());
-    for (int j = 0; j < nplanes; ++j)
-        CS_HIP(hipMemcpyAsync(outs[j], (Out*)dev.get() + j * n, sizeof(Out) * n, hipMemcpyDeviceToHost, l->stream));
-    CS_HIP(hipStreamSynchronize(l->stream));
+    planes_to_host((const Out*)dev.get(), n, outs, nplanes, l->stream);
 }
 
 static void reduce(cs_lattice* l, int nv, double* out_host)

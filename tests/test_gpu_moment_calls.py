@@ -1,0 +1,57 @@
+"""The moment calls' way to the host: a small lattice's planes cross in one
+copy, and what a call keeps on the device is bounded."""
+import time
+
+import numpy as np
+import pytest
+
+from chemsim_amd import Lattice, Params, capi
+from chemsim_amd import workloads as W
+from chemsim_amd.batch import Batch
+
+pytestmark = pytest.mark.gpu
+
+
+def _median_us(call, n=300):
+    call()
+    t = []
+    for _ in range(n):
+        t0 = time.perf_counter()
+        call()
+        t.append(time.perf_counter() - t0)
+    return 1e6 * float(np.median(t))
+
+
+def test_small_planes_take_one_copy(ctx):
+    """Three planes of 16 x 16 cost about what one costs (25 us; with a copy
+    and its latency per plane they took twice as long)."""
+    n = 16
+    ptr = lambda a: a.ctypes.data_as(capi.C.c_void_p)  # noqa: E731
+    f32, f64 = np.empty((3, n, n), np.float32), np.empty((3, n, n))
+    with Lattice(ctx, n, n, "f32", Params(tau=0.8)) as lat, Batch(ctx, [(n, n)], "f32") as b:
+        lat.init_equilibrium(*W.rest_state(n, n))
+        b.init_equilibrium(0, *W.rest_state(n, n))
+        one = _median_us(lambda: capi.call("cs_lattice_density", lat.handle, ptr(f32[0])))
+        three = _median_us(lambda: capi.call("cs_lattice_moments_f64", lat.handle, *(ptr(p) for p in f64)))
+        batch = _median_us(lambda: capi.call("cs_batch_moments", b.handle, 0, *(ptr(p) for p in f32)))
+    print(f"one plane {one:.1f} us, three {three:.1f} us, of a batch {batch:.1f} us")
+    assert three < 1.5 * one and batch < 1.5 * one
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 313, 443, 512])
+def test_planes_together_or_one_by_one(ctx, n):
+    """Either side of the bytes up to which planes cross together: every plane
+    lands in its own array, in the f32 and in the f64 calls."""
+    rng = np.random.default_rng(5)
+    rho = (1 + 0.01 * rng.standard_normal((n, n))).astype(np.float32)
+    u = (0.03 * rng.standard_normal((2, n, n))).astype(np.float32)
+    with Lattice(ctx, n, n, "f32", Params(tau=0.8)) as lat, Batch(ctx, [(n, n)], "f32") as b:
+        lat.init_equilibrium(rho, u[0], u[1])
+        b.init_equilibrium(0, rho, u[0], u[1])
+        f64 = lat.moments_f64()
+        ux, uy = lat.velocity()
+        for got in ((lat.density(), ux, uy), b.moments(0), (lat.density(), *b.velocity(0))):
+            for g, ref in zip(got, f64):
+                np.testing.assert_array_equal(g, ref.astype(np.float32))
+    np.testing.assert_allclose(f64[0], rho, rtol=1e-5)
+    np.testing.assert_allclose(f64[1:], u, atol=1e-6)
