@@ -210,7 +210,8 @@ struct cs_ctx {
 };
 
 struct cs_lattice {
-    cs_ctx* ctx = nullptr;
+    cs_ctx* ctx = nullptr;      // may be gone while the lattice steps: the kernel choice reads cus
+    int cus = 0;                // the device's compute units
     int w = 0, h = 0, storage = CS_F32;
     // Populations are row-interleaved: row r holds planes 0..8 of that row
     // one after another, so element (i, r, c) is at i * plane + r * pitch + c

@@ -788,6 +788,7 @@ extern "C" int cs_lattice_create(cs_ctx* ctx, int w, int h, int storage, cs_latt
         CS_HIP(hipSetDevice(ctx->device));
         auto* l = new cs_lattice;
         l->ctx = ctx;
+        l->cus = std::max(1, ctx->prop.multiProcessorCount);
         l->w = w;
         l->h = h;
         l->storage = storage;

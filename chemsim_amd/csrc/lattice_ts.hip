@@ -89,7 +89,7 @@ bool ts_takes(const cs_lattice* l)
     const bool half = l->has_flags && l->params.boundary == CS_BB_HALFWAY;
     const TsSplit s = ts_split(l, V, K);
     // both waves of (nearly) every SIMD, or the region kernels' many small blocks win
-    if (s.waves() < 6 * (int64_t)l->ctx->prop.multiProcessorCount) return false;
+    if (s.waves() < 6 * (int64_t)l->cus) return false;
     const double rows = (double)l->h / s.chunks;
     const double stream = (double)s.strips * 64 * V * (rows + K - 1) / ((double)l->w * rows);
     if (storage_bytes(l->storage) == 2) {

@@ -29,7 +29,7 @@ inline TsSplit ts_split(const cs_lattice* l, int v, int k)
     const int in = 64 * v - 2 * k;
     TsSplit s;
     s.strips = (l->w + in - 1) / in;
-    const int waves = 2 * 4 * std::max(1, l->ctx->prop.multiProcessorCount), most = (l->h + 7) / 8;
+    const int waves = 2 * 4 * l->cus, most = (l->h + 7) / 8;
     const bool walls = l->has_flags && l->params.boundary == CS_BB_HALFWAY && l->params.edge == CS_EDGE_ZERO;
     // an edge strip's time per row in inner strips': cavity and channel 4096^2,
     // GLUPS with 1, 1.3, 1.6, 2: 206, 226, 243, 242 and 181, 195, 192, 188
