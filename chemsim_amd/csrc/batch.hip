@@ -481,7 +481,7 @@ struct cs_batch {
     std::vector<unsigned char> host_lats;  // BatchLat<T> descriptors
     std::vector<LatState> host_state;     // `state` as of the launch
     cs_batch_tuning tuning{256, 2, 1, CS_ORDER_LARGEST_FIRST, CS_LAUNCH_PERSISTENT};
-    KeptStaging staging;              // result planes of the moment calls
+    std::shared_ptr<KeptStaging> staging;  // the context's: result planes of the moment calls
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
@@ -956,6 +956,7 @@ extern "C" int cs_batch_create(cs_ctx* ctx, int count, const int32_t* w, const i
         CS_HIP(hipSetDevice(ctx->device));
         auto* b = new cs_batch;
         b->ctx = ctx;
+        b->staging = ctx->staging();
         b->n = count;
         b->storage = storage;
         b->esize = storage_bytes(storage);
@@ -1032,8 +1033,7 @@ extern "C" int cs_batch_destroy(cs_batch* b)
         if (!b) return;
         if (b->stream) (void)hipStreamSynchronize(b->stream);
         for (void* p : {b->arena, (void*)b->nodes, b->d_lats, (void*)b->d_order, (void*)b->d_queue, (void*)b->snap,
-                        (void*)b->d_res, (void*)b->d_tiles, (void*)b->d_regions, (void*)b->d_bar, (void*)b->d_state,
-                        b->staging.p})
+                        (void*)b->d_res, (void*)b->d_tiles, (void*)b->d_regions, (void*)b->d_bar, (void*)b->d_state})
             if (p) (void)hipFree(p);
         if (b->ev0) (void)hipEventDestroy(b->ev0);
         if (b->ev1) (void)hipEventDestroy(b->ev1);
@@ -1201,7 +1201,7 @@ static void batch_moments(cs_batch* b, int index, unsigned mask, std::initialize
 {
     const size_t i = (size_t)index;
     const int64_t n = (int64_t)b->w[i] * b->h[i];
-    Staging dev(b->staging, sizeof(float) * (size_t)n * outs.size());
+    Staging dev(*b->staging, sizeof(float) * (size_t)n * outs.size(), b->stream);
     dispatch_batch_storage(b->storage, [&]<class St>() {
         dim3 g((unsigned)((b->w[i] + 255) / 256), (unsigned)b->h[i]);
         hipLaunchKernelGGL((k_moments<St, float>), g, dim3(256), 0, b->stream,

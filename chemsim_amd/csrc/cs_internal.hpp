@@ -7,7 +7,9 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <memory>
+#include <mutex>
 #include <string>
 
 #include "../../include/chemsim.h"
@@ -115,27 +117,41 @@ inline bool is_solid_flag(int t) { return t == CS_WALL || t == CS_LID; }
 
 size_t storage_bytes(int storage);
 
-// Device staging of a call's result planes.  A handle keeps one of up to
-// STAGING_KEEP bytes from call to call (hipMalloc and hipFree of a 2 MB
-// buffer take about as long as copying it to the host); larger requests are
-// allocated for the call.  Every user synchronises its stream before it returns.
+// Device staging of the moment calls' result planes: one buffer of up to
+// STAGING_KEEP bytes kept from call to call (hipMalloc and hipFree of a 2 MB
+// buffer take about as long as copying it to the host), shared by the handles
+// of a context and freed with the last of them -- one per handle would hold 12
+// to 24 bytes per cell of every lattice that was ever read.
+// A call that finds it taken by another thread's, or needs more, allocates its
+// own for the call.
 constexpr size_t STAGING_KEEP = (size_t)64 << 20;
 struct KeptStaging {
+    std::mutex mu;  // held by the call that uses the buffer
     void* p = nullptr;
     size_t bytes = 0;
+    KeptStaging() = default;
+    KeptStaging(const KeptStaging&) = delete;
+    KeptStaging& operator=(const KeptStaging&) = delete;
+    ~KeptStaging()
+    {
+        if (p) (void)hipFree(p);
+    }
 };
 class Staging {
 public:
-    Staging(KeptStaging& kept, size_t bytes)
+    // For work on `stream`, which is waited for before the buffer is given back.
+    Staging(KeptStaging& kept, size_t bytes, hipStream_t stream) : stream_(stream)
     {
-        if (bytes > STAGING_KEEP) {
+        if (bytes <= STAGING_KEEP) lock_ = std::unique_lock<std::mutex>(kept.mu, std::try_to_lock);
+        if (!lock_.owns_lock()) {
             CS_HIP(hipMalloc(&own_, bytes));
             p_ = own_;
             return;
         }
         if (bytes > kept.bytes) {
             if (kept.p) (void)hipFree(kept.p);
-            kept = KeptStaging{};
+            kept.p = nullptr;
+            kept.bytes = 0;
             CS_HIP(hipMalloc(&kept.p, bytes));
             kept.bytes = bytes;
         }
@@ -143,6 +159,7 @@ public:
     }
     ~Staging()
     {
+        if (std::uncaught_exceptions() > 0) (void)hipStreamSynchronize(stream_);  // else its user has waited
         if (own_) (void)hipFree(own_);
     }
     Staging(const Staging&) = delete;
@@ -150,6 +167,8 @@ public:
     void* get() const { return p_; }
 
 private:
+    std::unique_lock<std::mutex> lock_;
+    hipStream_t stream_;
     void* p_ = nullptr;
     void* own_ = nullptr;
 };
@@ -207,6 +226,16 @@ void render_enqueue(cs_lattice* l, int mode, int overlay, uint8_t* d_out, int ch
 struct cs_ctx {
     int device = 0;
     hipDeviceProp_t prop{};
+    std::mutex staging_mu;
+    std::weak_ptr<cs::KeptStaging> staging_now;
+    // The staging of this context's handles: made for the first, freed with the last.
+    std::shared_ptr<cs::KeptStaging> staging()
+    {
+        std::lock_guard<std::mutex> lk(staging_mu);
+        auto s = staging_now.lock();
+        if (!s) staging_now = s = std::make_shared<cs::KeptStaging>();
+        return s;
+    }
 };
 
 struct cs_lattice {
@@ -239,7 +268,7 @@ struct cs_lattice {
     int* iscratch = nullptr;
     double time = 0.0;
     uint64_t steps = 0;         // fused steps taken (keys the stochastic rounding)
-    cs::KeptStaging staging;    // result planes of the moment calls
+    std::shared_ptr<cs::KeptStaging> staging;  // the context's: result planes of the moment calls
     void* render_buf = nullptr; // render pass scratch (fields, partials, RGB)
     // Launch-bound lattices replay captured runs of fused steps: one graph per
     // starting buffer parity, valid for the parameters, geometry and launch

@@ -676,7 +676,7 @@ static void moments_to_host(cs_lattice* l, unsigned mask, Out* const* outs)
 {
     const int nplanes = __builtin_popcount(mask);
     const int64_t n = (int64_t)l->w * l->h;
-    Staging dev(l->staging, sizeof(Out) * n * nplanes);
+    Staging dev(*l->staging, sizeof(Out) * n * nplanes, l->stream);
     dispatch_storage(l->storage, [&]<class St>() {
         hipLaunchKernelGGL((k_moments<St, Out>), cell_grid(l), dim3(256), 0, l->stream,
                            (const typename St::S*)l->buf[l->cur], l->w, l->h, l->pitch, l->plane, consts_of<St>(l),
@@ -788,6 +788,7 @@ extern "C" int cs_lattice_create(cs_ctx* ctx, int w, int h, int storage, cs_latt
         CS_HIP(hipSetDevice(ctx->device));
         auto* l = new cs_lattice;
         l->ctx = ctx;
+        l->staging = ctx->staging();
         l->cus = std::max(1, ctx->prop.multiProcessorCount);
         l->w = w;
         l->h = h;
@@ -833,7 +834,7 @@ extern "C" int cs_lattice_destroy(cs_lattice* l)
         if (!l) return;
         if (l->stream) (void)hipStreamSynchronize(l->stream);
         for (void* p : {l->buf[0], l->buf[1], (void*)l->flags, (void*)l->node, (void*)l->snap, (void*)l->partials,
-                        (void*)l->dscratch, (void*)l->iscratch, l->render_buf, l->staging.p})
+                        (void*)l->dscratch, (void*)l->iscratch, l->render_buf})
             if (p) (void)hipFree(p);
         clear_step_graphs(l);
         if (l->ev0) (void)hipEventDestroy(l->ev0);

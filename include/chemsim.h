@@ -23,7 +23,9 @@
  *    calls are synchronous; cs_lattice_step is asynchronous on the lattice's
  *    own HIP stream.  Calls on one handle are not re-entrant; different
  *    handles may be used from different threads.
- *  - Handles own their device memory; *_destroy frees it.
+ *  - Handles own their device memory; *_destroy frees it.  The lattices and
+ *    batches of a context share one buffer of at most 64 MiB for the results
+ *    of the moment calls, kept until the last of them is destroyed.
  */
 #ifndef CHEMSIM_H
 #define CHEMSIM_H

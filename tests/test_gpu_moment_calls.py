@@ -1,11 +1,12 @@
 """The moment calls' way to the host: a small lattice's planes cross in one
 copy, and what a call keeps on the device is bounded."""
+import threading
 import time
 
 import numpy as np
 import pytest
 
-from chemsim_amd import Lattice, Params, capi
+from chemsim_amd import Context, Lattice, Params, capi
 from chemsim_amd import workloads as W
 from chemsim_amd.batch import Batch
 
@@ -55,3 +56,74 @@ def test_planes_together_or_one_by_one(ctx, n):
                 np.testing.assert_array_equal(g, ref.astype(np.float32))
     np.testing.assert_allclose(f64[0], rho, rtol=1e-5)
     np.testing.assert_allclose(f64[1:], u, atol=1e-6)
+
+
+def _free_bytes():
+    free, total = capi.C.c_size_t(), capi.C.c_size_t()
+    hip = capi.C.CDLL("libamdhip64.so")
+    assert hip.hipMemGetInfo(capi.C.byref(free), capi.C.byref(total)) == 0
+    return free.value
+
+
+def test_calls_keep_one_bounded_buffer_per_context(ctx):
+    """Reading 40 lattices of 1024 x 512 and a batch keeps at most the 64 MiB
+    that one context's handles share (12.6 MB for each would be 500 MB), and
+    gives it back with the last handle."""
+    w, h = 1024, 512
+    other = Context(0)
+    lats = [Lattice(other, w, h, "f32", Params(tau=0.8)) for _ in range(40)]
+    batch = Batch(other, [(w, h)] * 3, "f32")
+    rest = W.rest_state(w, h)
+    for lat in lats:
+        lat.init_equilibrium(*rest)
+    for i in range(3):
+        batch.init_equilibrium(i, *rest)
+    lats[0].sync()
+    before = _free_bytes()
+    for lat in lats:
+        lat.moments_f64()
+    for i in range(3):
+        batch.moments(i)
+    kept = before - _free_bytes()
+    print(f"kept {kept / 2**20:.1f} MiB")
+    assert kept <= (64 + 4) << 20  # and the allocator's granularity
+    big = Lattice(other, 2200, 2200, "f32", Params(tau=0.8))  # 116 MB of planes: allocated for the call
+    with_big = _free_bytes()
+    big.moments_f64()
+    assert with_big - _free_bytes() <= 4 << 20
+    for x in (*lats, batch, big):
+        x.close()
+    assert _free_bytes() >= before + 40 * 2 * 9 * 4 * w * h
+
+
+def test_moment_calls_from_several_threads(ctx):
+    """Lattices of one context read from several threads at once: the shared
+    buffer serves one call at a time, the others have their own."""
+    n, sides = 6, [64, 200, 333, 128, 512, 257]
+    lats, want = [], []
+    rng = np.random.default_rng(9)
+    for s in sides:
+        lat = Lattice(ctx, s, s, "f32", Params(tau=0.8))
+        lat.init_equilibrium((1 + 0.01 * rng.standard_normal((s, s))).astype(np.float32),
+                             *(0.03 * rng.standard_normal((2, s, s))).astype(np.float32))
+        lats.append(lat)
+        want.append((lat.density(), *lat.velocity(), *lat.moments_f64()))
+    errors = []
+
+    def read(k):
+        try:
+            for _ in range(40):
+                got = (lats[k].density(), *lats[k].velocity(), *lats[k].moments_f64())
+                for g, r in zip(got, want[k]):
+                    np.testing.assert_array_equal(g, r)
+        except BaseException as e:  # reported below
+            errors.append((k, repr(e)[:300]))
+
+    threads = [threading.Thread(target=read, args=(k,)) for k in range(n)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for lat in lats:
+        lat.close()
+    assert not errors, errors
