@@ -255,6 +255,7 @@ struct cs_lattice {
     uint8_t* flags = nullptr;   // h*pitch flags (device) or null
     uint32_t* node = nullptr;   // h*pitch node info (device) or null
     bool has_flags = false;
+    bool has_io = false;        // the flags hold an inlet or outlet cell
     cs_params params{};
     cs::Consts<float> k32{};
     cs::Consts<double> k64{};

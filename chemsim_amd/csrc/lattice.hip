@@ -903,8 +903,11 @@ extern "C" int cs_lattice_set_flags(cs_lattice* l, const uint8_t* flags)
             return;
         }
         const int64_t cells = (int64_t)l->w * l->h;
-        for (int64_t d = 0; d < cells; ++d)
+        bool io = false;
+        for (int64_t d = 0; d < cells; ++d) {
             CS_REQUIRE(flags[d] <= CS_OUTLET, CS_ERR_ARG, "flag value out of range");
+            io = io || flags[d] >= CS_INLET;
+        }
         if (!l->flags) {
             const size_t cells = (size_t)l->cpitch * l->h;
             CS_HIP(hipMalloc(&l->flags, cells));
@@ -919,6 +922,7 @@ extern "C" int cs_lattice_set_flags(cs_lattice* l, const uint8_t* flags)
         CS_HIP(hipGetLastError());
         CS_HIP(hipStreamSynchronize(l->stream));
         l->has_flags = true;
+        l->has_io = io;
     });
 }
 

@@ -5,16 +5,27 @@
 // A strip of rows costs a fill of K - 1 rows whatever its length, so the
 // streaming kernel needs a lattice that keeps every SIMD busy with long runs;
 // the region kernels (lbm_tb.hpp) recompute a fixed share instead.  Both
-// shares are known before the launch, so the choice compares them: computed
-// cells per kept cell, the streaming kernel's times 1.12 (what its instruction
-// mix costs more per computed cell; the ratio of measured times to computed
-// cells at 1536^2 .. 8192^2 is 1.07 .. 1.14; with half-way walls, whose region
-// kernel keeps its cells in LDS, 0.96 .. 1).  FP32 Taylor-Green, GLUPS,
-// streaming / regions in registers: 1024^2 110 / 174, 1536^2 187 / 218,
-// 2048^2 198 / 194, 3072^2 263 / 228, 4096^2 306 / 242, 8192^2 350 / 254;
-// half-way cavity, streaming / regions in LDS: 1536^2 118 / 122, 2001 x 1499
-// 139 / 132, 2048^2 160 / 141, 4096^2 243 / 161, 8192^2 288 / 166; channel with
-// obstacles 2048^2 126 / 108, 4096^2 192 / 118.
+// shares are known before the launch, so the choice (strip_rule.hpp) compares
+// them: computed cells per kept cell, the streaming kernel's times what a cell
+// costs it more.  Without half-way walls 1.12 (the ratio of measured times to
+// computed cells at 1536^2 .. 8192^2 is 1.07 .. 1.14).  The half-way mode's
+// region kernel keeps its cells in LDS: 1 for a periodic edge (2% of random
+// cells solid, 1800 x 1700 242 -> 192 us per 8 steps); where the lattice's edge
+// is a wall 1 too (cavities, us per 8 steps in strips / regions: 1700 x 2100 170 /
+// 198, 1721 x 1542 148 / 153), 1.1 for three to five strips (250 x 15000 243 /
+// 245, with TRT 316 / 300), 0.95 where every strip is an edge strip (150 x 20000
+// 243 / 268), and 1.2 more where the last strip keeps so few columns that an
+// inner one holds edge cells (1800 x 1700 192 / 175, 1459 x 2302 217 / 177, 1793 x
+// 2600 264 / 255, 2360 x 3000 338 / 365); 1.19 with inlet or outlet cells, whose
+// Zou-He divisions run in every row of an edge strip (channels 2048^2 231 / 220,
+// 2003 x 2300 240 / 237, 1260 x 3561 247 / 237, 3051 x 1713 262 / 286, 3000^2 406 /
+// 463), and 1.3 more with such a last strip (1800 x 1700 235 / 175, 3361 x 3100
+// 563 / 540).  More waves than the device holds take a second, nearly empty round:
+// 229500 x 48 is 2050 strips on 2048 slots, 455 / 366.
+// FP32 Taylor-Green, GLUPS, streaming / regions in registers: 1024^2 110 / 174,
+// 1536^2 187 / 218, 2048^2 198 / 194, 3072^2 263 / 228, 4096^2 306 / 242, 8192^2
+// 350 / 254; half-way cavity, streaming / regions in LDS: 1536^2 118 / 122,
+// 2001 x 1499 139 / 132, 2048^2 160 / 141, 4096^2 243 / 161, 8192^2 288 / 166.
 //
 // FP64 has no region kernels (a region would not fit), and its one-step kernel
 // is bound by HBM at 144 bytes per cell update: GLUPS, streaming / one-step,
@@ -80,27 +91,8 @@ void ts_edge(cs_lattice* l, int k)
 
 namespace cs {
 
-bool ts_takes(const cs_lattice* l)
-{
-    constexpr int K = 8, V = ts_cells<float>();
-    if (l->params.collision == CS_COLL_KBC) return false;
-    if (l->h < 2 * K) return false;  // the kernel wraps a row index once
-    if (l->storage == CS_F64) return (int64_t)l->w * l->h >= (int64_t)1 << 20;
-    const bool half = l->has_flags && l->params.boundary == CS_BB_HALFWAY;
-    const TsSplit s = ts_split(l, V, K);
-    // both waves of (nearly) every SIMD, or the region kernels' many small blocks win
-    if (s.waves() < 6 * (int64_t)l->cus) return false;
-    const double rows = (double)l->h / s.chunks;
-    const double stream = (double)s.strips * 64 * V * (rows + K - 1) / ((double)l->w * rows);
-    if (storage_bytes(l->storage) == 2) {
-        const bool sr = l->params.rounding == CS_ROUND_STOCHASTIC;
-        return stream < (half ? 1.65 : !sr ? 2.2 : l->storage == CS_BF16DEV ? 1.9 : 1.45);
-    }
-    constexpr int IN = TB_EDGE - 2 * K;
-    const double regions = (double)((l->w + IN - 1) / IN) * ((l->h + IN - 1) / IN) * TB_EDGE * TB_EDGE /
-                           ((double)l->w * l->h);
-    return (half ? 1.0 : 1.12) * stream < regions;
-}
+static_assert(TS_REGION_EDGE == TB_EDGE && ts_cells<float>() == 2, "what strip_rule.hpp counts");
+bool ts_takes(const cs_lattice* l) { return ts_takes(strip_case(l)); }
 
 void launch_ts(cs_lattice* l, int k)
 {

@@ -2,11 +2,11 @@
 // by the units that instantiate it.
 #pragma once
 
-#include <algorithm>
 #include <type_traits>
 
 #include "cs_internal.hpp"
 #include "lbm_ts.hpp"
+#include "strip_rule.hpp"
 
 namespace cs {
 
@@ -15,30 +15,19 @@ namespace cs {
 template <class T>
 constexpr int ts_cells() { return sizeof(T) == 8 ? 1 : 2; }
 
-// Waves are independent and all resident at once, two per SIMD; rows are
-// split into as many runs as that allows, of at least 8 rows.  Where the
-// lattice's own edge is a wall (half-way mode, zero edge), every row of the
-// first and the last strip takes the geometry pulls and the edge masks, so
-// these strips get more and shorter runs.
-struct TsSplit {
-    int strips, chunks, edge_chunks;
-    int64_t waves() const { return (int64_t)std::max(0, strips - 2) * chunks + (int64_t)std::min(strips, 2) * edge_chunks; }
-};
-inline TsSplit ts_split(const cs_lattice* l, int v, int k)
+inline StripCase strip_case(const cs_lattice* l)
 {
-    const int in = 64 * v - 2 * k;
-    TsSplit s;
-    s.strips = (l->w + in - 1) / in;
-    const int waves = 2 * 4 * l->cus, most = (l->h + 7) / 8;
-    const bool walls = l->has_flags && l->params.boundary == CS_BB_HALFWAY && l->params.edge == CS_EDGE_ZERO;
-    // an edge strip's time per row in inner strips': cavity and channel 4096^2,
-    // GLUPS with 1, 1.3, 1.6, 2: 206, 226, 243, 242 and 181, 195, 192, 188
-    const double share = walls ? 1.6 : 1.0;
-    const int edges = std::min(s.strips, 2);
-    const double unit = waves / (s.strips - edges + edges * share);
-    s.chunks = std::clamp((int)unit, 1, most);
-    s.edge_chunks = std::clamp((int)(unit * share), 1, most);
-    return s;
+    StripCase c;
+    c.w = l->w;
+    c.h = l->h;
+    c.storage = l->storage;
+    c.cus = l->cus;
+    c.half = l->has_flags && l->params.boundary == CS_BB_HALFWAY;
+    c.zero_edge = l->params.edge == CS_EDGE_ZERO;
+    c.io = c.half && l->has_io;
+    c.stochastic = l->params.rounding == CS_ROUND_STOCHASTIC;
+    c.kbc = l->params.collision == CS_COLL_KBC;
+    return c;
 }
 
 template <class St, int EDGE, int MODE, int K, int COLL, bool SR = false>
@@ -46,7 +35,7 @@ void ts_launch(cs_lattice* l)
 {
     using T = typename St::T;
     constexpr int V = ts_cells<T>();
-    const TsSplit sp = ts_split(l, V, K);
+    const TsSplit sp = ts_split(strip_case(l), V, K);
     TsArgs<T, K> A{};
     A.a.fin = l->buf[l->cur];
     A.a.fout = l->buf[l->cur ^ 1];

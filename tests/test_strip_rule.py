@@ -1,0 +1,101 @@
+"""Which lattices take 8 steps per launch in strips (chemsim_amd/csrc/strip_rule.hpp):
+the rule's answers for lattices whose two routes were both timed.  Host
+arithmetic, compiled here without a GPU."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+HEADER = os.path.join(os.path.dirname(HERE), "chemsim_amd", "csrc", "strip_rule.hpp")
+STORAGE = {"f32": 0, "f64": 1, "bf16": 2, "f16": 3, "f32dev": 4}
+# geometry: half-way mode, zero edge, inlet/outlet, reference mask
+GEOMETRY = {"periodic": (0, 0, 0, 0), "cavity": (1, 1, 0, 0), "channel": (1, 1, 1, 0), "porous": (1, 0, 0, 0),
+            "mask": (0, 0, 0, 1), "mask, zero edge": (0, 1, 0, 1)}
+MAIN = """
+#include <cstdio>
+#include "%s"
+int main()
+{
+    cs::StripCase c;
+    int half, zero, io, mask, sr;
+    while (std::scanf("%%d %%d %%d %%d %%d %%d %%d %%d", &c.w, &c.h, &c.storage, &half, &zero, &io, &mask, &sr) == 8) {
+        c.half = half;
+        c.zero_edge = zero;
+        c.io = io;
+        c.stochastic = sr;
+        std::printf("%%d\\n", (int)cs::ts_takes(c));
+    }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rule")
+    src, exe = str(d / "rule.cpp"), str(d / "rule")
+    with open(src, "w") as f:
+        f.write(MAIN % HEADER)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-o", exe, src], check=True, timeout=120)
+
+    def ask(storage, geometry, w, h, stochastic=False):
+        half, zero, io, mask = GEOMETRY[geometry]
+        r = subprocess.run([exe], input=f"{w} {h} {STORAGE[storage]} {half} {zero} {io} {mask} {int(stochastic)}",
+                           capture_output=True, text=True, timeout=20, check=True)
+        return [int(x) for x in r.stdout.split()]
+    return ask
+
+
+# us per 8 steps in regions / in strips
+@pytest.mark.parametrize("geometry,w,h", [
+    ("channel", 1800, 1700),   # 175 / 235
+    ("channel", 1950, 2047),   # 207 / 224
+    ("channel", 2048, 2048),   # 220 / 231
+    ("channel", 2003, 2300),   # 237 / 240
+    ("channel", 517, 9100),    # 258 / 272
+    ("channel", 250, 15000),   # 237 / 287
+    ("channel", 150, 20000),   # 247 / 287
+    ("channel", 60, 60000),    # 362 / 415
+    ("channel", 1260, 3561),   # 236 / 247
+    ("channel", 3361, 3100),   # 540 / 563, one column in the last strip
+    ("channel", 1572, 3361),   # 281 / 354, four
+    ("cavity", 1800, 1700),    # 175 / 192, eight
+    ("cavity", 1353, 2300),    # 173 / 193, nine
+    ("cavity", 1459, 2302),    # 177 / 217, three
+    ("cavity", 1793, 2600),    # 255 / 264, one
+    ("cavity", 250, 15000),    # 245 / 243, TRT 300 / 316
+    ("cavity", 229500, 48),    # 607 / 638
+    ("periodic", 229500, 48),  # 366 / 455
+    ("periodic", 229500, 144),  # 1085 / 1217
+    ("periodic", 1024, 1024),
+    ("periodic", 1536, 1536),
+])
+@pytest.mark.parametrize("storage", ["f32", "f32dev"])
+def test_fp32_keeps_regions_where_they_are_faster(rule, storage, geometry, w, h):
+    assert rule(storage, geometry, w, h)[0] == 0
+
+
+@pytest.mark.parametrize("geometry,w,h", [
+    ("channel", 3000, 3000),   # 463 / 406
+    ("channel", 9100, 517),    # 259 / 227
+    ("channel", 101, 30011),   # 287 / 258
+    ("channel", 3369, 3100),   # 540 / 455, nine columns in the last strip
+    ("cavity", 2360, 3000),    # 365 / 338, eight
+    ("cavity", 1721, 1542),    # 153 / 148
+    ("cavity", 1700, 2100),    # 198 / 170
+    ("cavity", 2001, 1499),
+    ("cavity", 2048, 2048),    # 227 / 183
+    ("cavity", 517, 9100),     # 262 / 228
+    ("cavity", 150, 20000),    # 268 / 243
+    ("cavity", 49, 60000),     # 407 / 327
+    ("porous", 1800, 1700),    # 242 / 192
+    ("mask", 2500, 2000),      # 200 / 200
+    ("mask", 3000, 3000),      # 347 / 296
+    ("periodic", 2003, 2300),  # 161 / 148
+    ("periodic", 57400, 96),   # 197 / 179
+    ("periodic", 250000, 24),  # 381 / 268
+    ("periodic", 4096, 4096),
+])
+@pytest.mark.parametrize("storage", ["f32", "f32dev"])
+def test_fp32_takes_strips_where_they_are_faster(rule, storage, geometry, w, h):
+    assert rule(storage, geometry, w, h)[0] == 1
