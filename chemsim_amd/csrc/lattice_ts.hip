@@ -45,6 +45,20 @@
 // so f16 with stochastic rounding takes it only where the fill is small.
 // Half-way cavity 2048^2 and 4096^2: f16 148 / 99, 224 / 121 to nearest, 101 /
 // 95, 141 / 116 stochastic; bf16 111 / 94, 164 / 115 and 98 / 95, 138 / 118.
+// What else moves the line (us per 8 steps, streaming / one-step):
+//   wave slots left idle, since the one-step kernels fill the device whatever the
+//   shape: 57400 x 288 (513 strips, 3 runs each) f16 stochastic 1032 / 907, 229500
+//   x 96 bf16 to nearest 1350 / 1274; f16 to nearest is faster all the same, 975 /
+//   1262;
+//   inlets and outlets with stochastic rounding (f16 / bf16 2048^2 364 / 331, 379 /
+//   331; 3000^2 634 / 628, 659 / 627; 4096^2 1073 / 1131, 1121 / 1126);
+//   a solid mask: bf16 stochastic 2048^2 with a few obstacles 294 / 271, with 2%
+//   of random cells 306 / 272, 3000^2 520 / 536; bf16 to nearest 1500^2 182 / 170,
+//   1800 x 1700 220 / 223; f16 stochastic 4100 x 1517 396 / 382, 9100 x 817 466 / 468;
+//   a wall in an inner strip (FP32 above): bf16 stochastic cavity 2353 x 3000 577 /
+//   539, 3361 x 3100 779 / 737;
+// against the one-step kernels' tiles of 256 columns in these modes, which a
+// narrow lattice leaves half empty: 101 x 30011 channel bf16 stochastic 375 / 417.
 #include "lattice_ts.hpp"
 #include "lbm_tb.hpp"
 

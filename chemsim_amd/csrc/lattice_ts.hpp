@@ -25,6 +25,7 @@ inline StripCase strip_case(const cs_lattice* l)
     c.half = l->has_flags && l->params.boundary == CS_BB_HALFWAY;
     c.zero_edge = l->params.edge == CS_EDGE_ZERO;
     c.io = c.half && l->has_io;
+    c.mask = l->has_flags && !c.half;
     c.stochastic = l->params.rounding == CS_ROUND_STOCHASTIC;
     c.kbc = l->params.collision == CS_COLL_KBC;
     return c;

@@ -18,6 +18,7 @@ struct StripCase {
     bool half = false;        // half-way boundary mode with flags
     bool zero_edge = false;   // zero edge, not periodic
     bool io = false;          // ... and inlet or outlet cells
+    bool mask = false;        // reference boundary mode with flags
     bool stochastic = false;  // 16-bit storage: stochastic rounding
     bool kbc = false;
     bool walls() const { return half && zero_edge; }  // the lattice's own edge is a wall
@@ -97,14 +98,24 @@ inline bool ts_takes_32(const StripCase& c)
     return cost * two * computed * (s.waves() > 8 * (int64_t)c.cus ? 1 + 0.6 * (idle - 1) : 1) < regions;
 }
 
-// 16-bit storage: strips against the one-step kernels.
+// 16-bit storage: strips against the one-step kernels, whose geometry modes
+// compute whole tiles of 256 columns.
 inline bool ts_takes_16(const StripCase& c)
 {
     constexpr int K = 8;
     const bool bf16 = c.storage == CS_BF16DEV, sr = c.stochastic;
     const double stream = ts_computed(c, K);
     const double most = c.half ? 1.65 : !sr ? 2.2 : bf16 ? 1.9 : 1.45;
-    return stream < most;
+    if (stream >= most) return false;
+    if (!bf16 && !sr) return true;
+    const double idle = ts_idle(c, ts_split(c, 2, K).waves());
+    const double cost = stream * (1 + (bf16 || c.half ? 1.5 : 1.0) * std::max(0.0, idle - 1.05)) *
+                        (ts_two_wall_strips(c) ? 1.3 : 1.0);
+    const double tiles = (double)((c.w + 255) / 256 * 256) / c.w;
+    if (c.io && sr) return cost / tiles < 1.31;
+    if (c.half) return cost < (sr ? most : 2.0);
+    if (c.mask) return cost / tiles < (!sr ? 1.75 : bf16 ? 1.375 : 1.4);
+    return cost < most;
 }
 
 // Whether the lattice takes 8 steps per launch in strips.  The figures behind

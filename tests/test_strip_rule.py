@@ -23,6 +23,7 @@ int main()
         c.half = half;
         c.zero_edge = zero;
         c.io = io;
+        c.mask = mask;
         c.stochastic = sr;
         std::printf("%%d\\n", (int)cs::ts_takes(c));
     }
@@ -99,3 +100,56 @@ def test_fp32_keeps_regions_where_they_are_faster(rule, storage, geometry, w, h)
 @pytest.mark.parametrize("storage", ["f32", "f32dev"])
 def test_fp32_takes_strips_where_they_are_faster(rule, storage, geometry, w, h):
     assert rule(storage, geometry, w, h)[0] == 1
+
+
+# us per 8 steps in one-step launches / in strips
+@pytest.mark.parametrize("storage,stochastic,geometry,w,h", [
+    ("bf16", True, "mask", 2048, 2048),      # 271 / 294 with six obstacles, 272 / 306 with 2% solid
+    ("bf16", True, "mask", 2500, 2000),      # 319 / 338, 321 / 346
+    ("bf16", True, "mask", 1800, 1700),      # 223 / 245, 224 / 256
+    ("bf16", False, "mask", 1500, 1500),     # 173 / 178, 170 / 182
+    ("bf16", False, "mask", 250, 15000),     # 265 / 280 with 2% solid
+    ("f16", True, "mask", 57400, 144),       # 489 / 569
+    ("f16", True, "channel", 2048, 2048),    # 330 / 363
+    ("bf16", True, "channel", 2048, 2048),   # 329 / 379
+    ("bf16", True, "channel", 3000, 3000),   # 627 / 659
+    ("bf16", True, "cavity", 2353, 3000),    # 539 / 577, one column in the last strip
+    ("f16", True, "cavity", 2353, 3000),     # 540 / 555
+    ("bf16", True, "cavity", 3361, 3100),    # 737 / 779
+    ("f16", True, "cavity", 57400, 288),     # 1107 / 1157
+    ("bf16", True, "cavity", 400000, 17),    # 540 / 612
+    ("f16", True, "cavity", 400000, 17),     # 540 / 570
+    ("bf16", False, "cavity", 250000, 32),   # 569 / 723
+    ("bf16", False, "periodic", 250000, 32),  # 473 / 528
+    ("bf16", True, "periodic", 229500, 96),  # 1271 / 1515
+    ("f16", True, "periodic", 57400, 288),   # 907 / 1032
+    ("f16", True, "periodic", 60001, 120),   # 434 / 475
+    ("f16", True, "periodic", 2048, 2048),
+])
+def test_16bit_keeps_single_steps_where_they_are_faster(rule, storage, stochastic, geometry, w, h):
+    assert rule(storage, geometry, w, h, stochastic)[0] == 0
+
+
+@pytest.mark.parametrize("storage,stochastic,geometry,w,h", [
+    ("bf16", True, "mask", 3000, 3000),      # 536 / 520 with 2% solid
+    ("bf16", True, "mask", 9100, 817),       # 464 / 433, 469 / 465
+    ("bf16", False, "mask", 2048, 2048),     # 275 / 262 with 2% solid
+    ("bf16", False, "mask", 101, 30011),     # 273 / 223
+    ("f16", False, "mask", 1800, 1700),      # 214 / 173
+    ("f16", True, "mask", 4096, 4096),       # 1001 / 906
+    ("f16", True, "channel", 4096, 4096),    # 1131 / 1073
+    ("f16", True, "channel", 101, 30011),    # 417 / 367
+    ("bf16", True, "channel", 517, 9100),    # 440 / 411
+    ("bf16", False, "channel", 2048, 2048),  # 334 / 330
+    ("f16", False, "channel", 2048, 2048),   # 320 / 256
+    ("f16", True, "cavity", 2048, 2048),     # 347 / 324
+    ("bf16", False, "cavity", 57400, 144),   # 582 / 548
+    ("f16", True, "porous", 1950, 2047),     # 422 / 336
+    ("f16", False, "periodic", 229500, 96),  # 1262 / 975
+    ("bf16", True, "periodic", 1800, 1700),  # 220 / 199
+    ("f16", True, "periodic", 4096, 4096),   # 892 / 837
+    ("f16", True, "periodic", 21280, 800),
+    ("bf16", False, "periodic", 70, 90011),  # 624 / 383
+])
+def test_16bit_takes_strips_where_they_are_faster(rule, storage, stochastic, geometry, w, h):
+    assert rule(storage, geometry, w, h, stochastic)[0] == 1
