@@ -153,6 +153,7 @@ int tb_remainder_plan(const cs_lattice* l, int plan)
 {
     if (storage_bytes(l->storage) == 2) return 0;
     if (tb_plan_steps(plan) != 8 || l->params.collision != CS_COLL_BGK) return 0;
+    if ((plan >> 8) == TS_PLAN && !ts_takes_remainder(l)) return tb_plan(4, TB_EDGE);
     return (plan & ~0xFF) | 4;
 }
 

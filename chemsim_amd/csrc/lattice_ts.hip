@@ -59,6 +59,14 @@
 //   539, 3361 x 3100 779 / 737;
 // against the one-step kernels' tiles of 256 columns in these modes, which a
 // narrow lattice leaves half empty: 101 x 30011 channel bf16 stochastic 375 / 417.
+//
+// A 4-step remainder launch recomputes less in strips and in regions alike (a
+// 64 x 64 region keeps 56 x 56), so its line is its own: us per 4 steps, strips /
+// regions, 4096^2 309 / 337, 1794 x 3541 126 / 130, 2893 x 1432 95 / 91, 1100 x 4003
+// 92 / 91; with a solid mask 3000^2 190 / 202, 1780 x 2635 108 / 102, 1100 x 4003
+// 103 / 96; cavity 2048^2 101 / 140, 49 x 60000 (one region wide) 164 / 148,
+// channel 201 / 143; 101 x 30011 (one strip) 79 / 83.  FP64, which has no
+// regions: 0.35 to 0.55 of four single steps.
 #include "lattice_ts.hpp"
 #include "lbm_tb.hpp"
 
@@ -107,6 +115,7 @@ namespace cs {
 
 static_assert(TS_REGION_EDGE == TB_EDGE && ts_cells<float>() == 2, "what strip_rule.hpp counts");
 bool ts_takes(const cs_lattice* l) { return ts_takes(strip_case(l)); }
+bool ts_takes_remainder(const cs_lattice* l) { return ts_takes_remainder(strip_case(l)); }
 
 void launch_ts(cs_lattice* l, int k)
 {

@@ -131,4 +131,13 @@ inline bool ts_takes(const StripCase& c)
     return c.storage == CS_BF16DEV || c.storage == CS_F16DEV ? ts_takes_16(c) : ts_takes_32(c);
 }
 
+// A lattice of 8 steps per launch in strips: whether its 4-step remainder
+// launch goes in strips too, or (FP32) in regions.
+inline bool ts_takes_remainder(const StripCase& c)
+{
+    if (c.storage == CS_F64) return true;
+    const bool narrow = ts_split(c, 2, 4).strips <= 2;
+    return ts_computed(c, 4) < (c.half ? 1.2 : narrow ? 1.1 : c.mask ? 0.907 : 0.96) * region_computed(c, 4);
+}
+
 }  // namespace cs

@@ -25,7 +25,7 @@ int main()
         c.io = io;
         c.mask = mask;
         c.stochastic = sr;
-        std::printf("%%d\\n", (int)cs::ts_takes(c));
+        std::printf("%%d %%d\\n", (int)cs::ts_takes(c), (int)cs::ts_takes_remainder(c));
     }
 }
 """
@@ -153,3 +153,25 @@ def test_16bit_keeps_single_steps_where_they_are_faster(rule, storage, stochasti
 ])
 def test_16bit_takes_strips_where_they_are_faster(rule, storage, stochastic, geometry, w, h):
     assert rule(storage, geometry, w, h, stochastic)[0] == 1
+
+
+# us per 4 steps in regions / in strips, of lattices that take strips for 8
+@pytest.mark.parametrize("geometry,w,h,strips", [
+    ("cavity", 49, 60000, 0),       # 148 / 164
+    ("cavity", 150, 20000, 0),      # 123 / 118; channel 126 / 140
+    ("cavity", 2048, 2048, 1),      # 140 / 101
+    ("cavity", 517, 9100, 1),       # 157 / 134
+    ("channel", 3000, 3000, 1),     # 308 / 220
+    ("periodic", 2893, 1432, 0),    # 91 / 95
+    ("periodic", 1100, 4003, 0),    # 91 / 92
+    ("periodic", 1794, 3541, 1),    # 130 / 126
+    ("periodic", 4096, 4096, 1),    # 337 / 309
+    ("periodic", 101, 30011, 1),    # 83 / 79
+    ("mask", 1848, 2434, 0),        # 99 / 105
+    ("mask", 1780, 2635, 0),        # 102 / 108
+    ("mask", 1491, 3577, 0),        # 116 / 122
+    ("mask", 3202, 1526, 0),        # 114 / 118
+    ("mask", 3000, 3000, 1),        # 202 / 190
+])
+def test_remainder_takes_the_faster_of_both(rule, geometry, w, h, strips):
+    assert rule("f32", geometry, w, h) == [1, strips]
