@@ -116,10 +116,6 @@ struct TsLds {
 template <class T, int K, int V>
 struct TsLds<T, MODE_FLUID, K, V> {};
 
-constexpr int ts_up(int q) { return q == 0 ? 1 : (q == 1 ? 5 : 8); }   // pulled from the row below (r + 1)
-constexpr int ts_mid(int q) { return q == 0 ? 0 : (q == 1 ? 2 : 4); }  // from the row itself
-constexpr int ts_dn(int q) { return q == 0 ? 3 : (q == 1 ? 6 : 7); }   // from the row above (r - 1)
-
 // One strip and chunk: output rows ra .. rb-1, columns c0 + K .. c0 + 64 V - K - 1.
 template <class St, int EDGE, int MODE, int K, int COLL, int V, bool SR>
 __device__ __forceinline__ void ts_strip(const TsArgs<typename St::T, K>& A, int c0, int ra, int rb,
