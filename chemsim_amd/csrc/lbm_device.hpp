@@ -224,7 +224,11 @@ __device__ __forceinline__ float recip_rn<float>(float b)
 // of a SIMD from issuing side by side for about a thousand cycles after it
 // (measured: add/mul streams of two waves 0.46 wave instructions per SIMD and
 // cycle, with one v_rcp_f32 in 256 instructions 0.26).  Newton-Raphson from
-// the integer estimate magic - bits(b) (within 6%): a cubic step, y (1 + e +
+// the integer estimate M - bits(b): with b = 2^k (1 + m) and M = (254 - d) 2^23
+// its product with b is (1 + m)(2 - m - d) / 2 up to m = 1 - d and (1 + m)(3 - m -
+// d) / 4 from there, between 1 - d / 2 and (3 - d)^2 / 8.  The two are equally
+// far from 1 for d^2 - 10 d + 1 = 0, d = 5 - sqrt(24) = 0.10102 (847421 units of
+// 2^-23), which makes the estimate good to 5.06%.  A cubic step, y (1 + e +
 // e^2) with e = 1 - b y, brings it to 2e-4, a quadratic one to an ulp, and the
 // last, y + y e with e exact, is the FMA reciprocal iteration of P. W.
 // Markstein, "Computation of elementary functions on the IBM RISC System/6000
@@ -237,7 +241,7 @@ __device__ __forceinline__ float recip_rn<float>(float b)
 __device__ __forceinline__ float recip_newton(float b, bool& ok)
 {
     const uint32_t x = __builtin_bit_cast(uint32_t, b);
-    float y = __builtin_bit_cast(float, 0x7EF311C7u - x);
+    float y = __builtin_bit_cast(float, 0x7F000000u - 847421u - x);
     float e = __builtin_fmaf(-b, y, 1.0f);
     y = __builtin_fmaf(__builtin_fmaf(e, e, e), y, y);
     e = __builtin_fmaf(-b, y, 1.0f);
