@@ -304,6 +304,7 @@ struct Act {
 
 struct cs_cnn {
     cs_ctx* ctx = nullptr;
+    int cus = 0;                      // the device's compute units
     int H = 0, W = 0, base = 0, batch = 0;
     hipStream_t stream = nullptr;
     std::vector<Conv> convs;          // 19 convolutions in forward order
@@ -390,7 +391,7 @@ void gemm(cs_cnn* net, int la, int lb, int epi, const uint16_t* A, int lda, cons
     CS_REQUIRE(K % 8 == 0, CS_ERR_ARG, "gemm K must be a multiple of 8");
     g.k_per_split = ((K + splits - 1) / splits + BK - 1) / BK * BK;  // splits cover [0, K)
     g.split_stride = (int64_t)M * ldc;
-    const int cfg = la == GATHER && splits == 1 ? pick_gather_tile(M, N) : pick_tile(M, N);
+    const int cfg = la == GATHER && splits == 1 ? pick_gather_tile(M, N, net->cus) : pick_tile(M, N);
     int bm, bn;
     tile_dims(cfg, bm, bn);
     dim3 grid((unsigned)((M + bm - 1) / bm), (unsigned)((N + bn - 1) / bn), (unsigned)splits);
@@ -441,7 +442,7 @@ void conv_halo(cs_cnn* net, int epi, const Act& x, const uint16_t* w, int ldw, c
     // output's sums does not depend on it): one 128 x 512 image predicted in 0.62 ms
     // without, 0.58 / 0.56 / 0.55 ms at 128 / 256 / 512 blocks; two images' training
     // step 1.42 -> 1.31 ms
-    while (bn > 16 && tiles * ((N + bn - 1) / bn) < 512) bn /= 2;
+    while (bn > 16 && tiles * ((N + bn - 1) / bn) < 2 * net->cus) bn /= 2;
     const dim3 grid((unsigned)tiles, (unsigned)((N + bn - 1) / bn));
     net->gemm_flops += 2.0 * (double)x.P() * N * kflops;
     auto go = [&]<int EPI>() {
@@ -715,6 +716,7 @@ extern "C" int cs_cnn_create(cs_ctx* ctx, int height, int width, int base, int b
         auto* net = new cs_cnn;
         try {
             net->ctx = ctx;
+            net->cus = std::max(1, ctx->prop.multiProcessorCount);
             net->H = height;
             net->W = width;
             net->base = base;

@@ -414,13 +414,13 @@ inline void tile_dims(int cfg, int& bm, int& bn)
 // one channel 785 -> 605 us, training step of eight 3.03 -> 2.92 ms.  The
 // accumulation order of an output does not depend on the tile.  (Two to four K
 // slices in flight instead of one measured the same.)
-inline int pick_gather_tile(int M, int N)
+inline int pick_gather_tile(int M, int N, int cus)
 {
     const int cfg = pick_tile(M, N);
     if (cfg != TILE_128x128) return cfg;
     const auto blocks = [&](int t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t); };
-    if (blocks(128) >= 256) return TILE_128x128;
-    return blocks(64) >= 256 ? TILE_64x64 : TILE_32x32;
+    if (blocks(128) >= cus) return TILE_128x128;
+    return blocks(64) >= cus ? TILE_64x64 : TILE_32x32;
 }
 
 template <int LA, int LB, int EPI>
