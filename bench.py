@@ -4,8 +4,8 @@ Default workload: periodic Taylor-Green vortex, 4096 x 4096, FP32, tau = 0.8,
 u0 = 0.05, wavenumber 2 pi / 4096; K timed steps after W warm-up steps, with
 the populations resident in HBM.  A step is one full update (stream +
 bounce-back + BGK collide) of every cell.  FP32 lattices take the temporally
-blocked kernel (8 steps per launch with the region in registers; a remainder
-of 4 or more steps one 4-step launch, the rest one step per launch); the
+blocked kernels (8 steps per launch, in strips or regions as the library chooses;
+a remainder of 4 or more steps one 4-step launch, the rest one step per launch); the
 one-step kernel of the same workload is timed beside it in `extras`.  Before
 the warm-up, each kernel the timed steps use is launched once on a scratch
 lattice of the same shape, so first-launch costs stay out of the timed region
@@ -16,10 +16,9 @@ region a scratch lattice's steps keep the GPU busy for 0.05 s (wake_gpu);
 Prints ONE JSON line.  `value` is lattice updates per second (GLUPS) over the
 timed steps (wall clock around a synchronised region); the roofline object
 prices the step kernel's average duration (HIP events on the lattice's own
-stream) against the bytes that kernel must move: for the temporally blocked
-kernel each 64 x 64 region (interior and halo) read once and each interior
-cell written once per launch, for the one-step kernels 72 bytes per cell
-update.  The CPU baseline is the oracle's fused FP32 step (OpenMP over rows)
+stream) against the bytes that its launches cannot do without: the lattice read
+once and written once per launch, 72 bytes per cell for FP32, whether a launch
+makes 8 steps, 4 or one.  The CPU baseline is the oracle's fused FP32 step (OpenMP over rows)
 on a bounded sample of the same lattice.
 """
 from __future__ import annotations
@@ -60,64 +59,27 @@ def tb_region_edge(w: int, h: int) -> int:
 
 
 def tb_bytes_per_step(w: int, h: int, esize: int = 4, k: int = TB_STEPS, edge: int | None = None) -> float:
-    """Bytes one launch of the temporally blocked kernel must move, per step:
-    every region (interior of side edge - 2k plus halo) read once, every
-    lattice cell written once, 9 populations of `esize` bytes.  `edge`: the
-    region side (default: the single-lattice choice; batches use 64)."""
+    """Bytes one launch of the region kernels requests, per step: every region
+    (interior of side edge - 2k plus halo) read once, every lattice cell written
+    once, 9 populations of `esize` bytes.  `edge`: the region side (default: the
+    single-lattice choice; batches use 64)."""
     edge = tb_region_edge(w, h) if edge is None else edge
     inner = edge - 2 * k
     regions = -(-w // inner) * -(-h // inner)
     return (regions * edge * edge + w * h) * 9 * esize / k
 
 
-def ts_split(w: int, h: int, storage: str, k: int = TB_STEPS) -> tuple[int, int, int]:
-    """Columns per strip, strips and runs of rows per strip of the streaming
-    kernel on a lattice without walls (two waves per SIMD of 256 CUs)."""
-    cols = 64 if storage == "f64" else 128
-    strips = -(-w // (cols - 2 * k))
-    return cols, strips, max(1, min(2048 // strips, (h + 7) // 8))
-
-
-def ts_takes(w: int, h: int, storage: str, rounding: str = "sr") -> bool:
-    """Whether a periodic BGK lattice takes the streaming kernel (the rule of
-    chemsim_amd/csrc/lattice_ts.hip)."""
-    if h < 16:
-        return False
-    if storage == "f64":
-        return w * h >= 1 << 20
-    cols, strips, chunks = ts_split(w, h, storage)
-    if strips * chunks < 1536:
-        return False
-    rows = h / chunks
-    stream = strips * cols * (rows + TB_STEPS - 1) / (w * rows)
-    if storage in ("f16", "bf16"):
-        return stream < (2.2 if rounding != "sr" else 1.9 if storage == "bf16" else 1.45)
-    inner = TB_EDGE - 2 * TB_STEPS
-    return 1.12 * stream < -(-w // inner) * -(-h // inner) * TB_EDGE * TB_EDGE / (w * h)
-
-
-def ts_bytes_per_step(w: int, h: int, storage: str, k: int = TB_STEPS) -> float:
-    """Bytes one launch of the streaming kernel must move, per step: every run
-    reads its rows and k more on either side over the strip's columns, every
-    lattice cell is written once."""
-    cols, strips, chunks = ts_split(w, h, storage, k)
-    return (strips * cols * (h + 2 * k * chunks) + w * h) * BYTES_PER_CELL[storage] / 2 / k
-
-
-def step_bytes_per_cell(storage: str, n: int, k: int, rounding: str = "sr") -> float:
-    """Algorithmic bytes per cell update of the kernel an n x n lattice takes
-    (k: steps per launch, Lattice.temporal_steps(); 1 = a one-step kernel)."""
-    if k > 1:
-        if ts_takes(n, n, storage, rounding):
-            return ts_bytes_per_step(n, n, storage, k) / (n * n)
-        return tb_bytes_per_step(n, n, k=k) / (n * n)
-    return BYTES_PER_CELL[storage]
+def step_bytes_per_cell(storage: str, k: int) -> float:
+    """Bytes per cell update that k steps per launch cannot do without: one read
+    and one write of the 9 populations per launch, in whichever kernel (halo
+    cells read again are extra, mostly served by the caches)."""
+    return BYTES_PER_CELL[storage] / k
 
 
 def run_bytes_per_cell(storage: str, n: int, k: int, steps: int) -> float:
-    """Algorithmic bytes per cell update of a run of `steps` BGK steps on an
-    n x n lattice: the k-step launches, then (k = 8) one 4-step launch for a
-    remainder of 4 or more steps, then one-step launches."""
+    """Bytes per cell update that the region kernels request over a run of
+    `steps` BGK steps on an n x n lattice: the k-step launches, then (k = 8) one
+    4-step launch for a remainder of 4 or more steps, then one-step launches."""
     if k <= 1:
         return BYTES_PER_CELL[storage]
     nk, r = divmod(steps, k)
@@ -128,17 +90,14 @@ def run_bytes_per_cell(storage: str, n: int, k: int, steps: int) -> float:
     return total / (n * n * steps)
 
 
-def launched_bytes_per_cell(storage: str, n: int, k: int, steps: int) -> float:
-    """run_bytes_per_cell with the streaming kernel's bytes where an n x n
-    lattice takes it (a remainder of 4 steps as one 4-step launch for 4- and
-    8-byte storage)."""
-    if k <= 1 or not ts_takes(n, n, storage):
-        return run_bytes_per_cell(storage, n, k, steps)
+def launched_bytes_per_cell(storage: str, k: int, steps: int) -> float:
+    """step_bytes_per_cell over the launches of a run of `steps` BGK steps: the
+    k-step launches, then (k = 8, 4- and 8-byte storage) one 4-step launch for a
+    remainder of 4 or more steps, then one-step launches."""
     nk, r = divmod(steps, k)
-    n4 = 1 if r >= 4 and BYTES_PER_CELL[storage] > 36 else 0
-    total = nk * k * ts_bytes_per_step(n, n, storage, k) + n4 * 4 * ts_bytes_per_step(n, n, storage, 4) \
-        + (r - 4 * n4) * n * n * BYTES_PER_CELL[storage]
-    return total / (n * n * steps)
+    n4 = 1 if k == 8 and r >= 4 and BYTES_PER_CELL[storage] > 36 else 0
+    launches = nk + n4 + (r - 4 * n4)
+    return launches * BYTES_PER_CELL[storage] / steps
 
 
 def warm_kernels(ctx, n, storage, tau, u0, rounding="sr"):
@@ -313,7 +272,7 @@ def tgv_8192_run(ctx, tau, u0, steps=200):
         r, x, y = lat.moments_f64()
         lat.close()
         out[st] = {"GLUPS": round(cells * steps / w / 1e9, 3), "kernel_us": round(ms / steps * 1e3, 1),
-                   "hbm_frac": hbm_frac(step_bytes_per_cell(st, n, k), cells, ms / steps), "steps_per_launch": k,
+                   "hbm_frac": hbm_frac(step_bytes_per_cell(st, k), cells, ms / steps), "steps_per_launch": k,
                    "u_rel_L2_vs_f64": float(np.sqrt(((x - x64) ** 2 + (y - y64) ** 2).sum()) / den),
                    "rho_dev_rel_L2_vs_f64": float(np.sqrt(((r - r64) ** 2).sum()) / rden)}
         del r, x, y
@@ -388,7 +347,7 @@ def batch_cavities_run(ctx, steps=5000, per_lattice_steps=20, other_steps=1000):
     b.tuning = best
     ms_pl = b.step_per_lattice(per_lattice_steps)
     cells = b.cells
-    # bytes the launch kind must move per cell update: 72 for one-step launches; for the
+    # bytes the launch kind requests per cell update: 72 for one-step launches; for the
     # temporal kind every 64 x 64 region read and every cell written once per 8 steps
     bpc = 72.0
     if best.get("launch", 0) in (capi.CS_LAUNCH_TEMPORAL, capi.CS_LAUNCH_TEMPORAL_PERSISTENT):
@@ -450,7 +409,7 @@ def main():
     kernel_ms = ms / args.steps
     k_launch = lat.temporal_steps()
     temporal = k_launch > 1
-    bpc = launched_bytes_per_cell(storage, n, k_launch, args.steps)
+    bpc = launched_bytes_per_cell(storage, k_launch, args.steps)
     achieved = bpc * cells / (kernel_ms * 1e-3) / 1e9
     log(f"[bench] {glups:.2f} GLUPS wall, {kernel_ms * 1e3:.1f} us/step (events), {achieved:.0f} GB/s algorithmic")
     # four more timed regions of the same length, for the spread (value stays the first)
@@ -489,7 +448,7 @@ def main():
                                      "kernel_us": round(ms1 / args.steps * 1e3, 2),
                                      "hbm_frac": hbm_frac(BYTES_PER_CELL[storage], cells, ms1 / args.steps),
                                      "bytes_per_cell": BYTES_PER_CELL[storage]}
-        extras["temporal_blocking"] = {"steps_per_launch": k_launch, "kernel": "streaming" if ts_takes(n, n, storage) else "regions",
+        extras["temporal_blocking"] = {"steps_per_launch": k_launch,
                                        "bytes_per_cell_update": round(bpc, 3),
                                        "speedup_vs_one_step": round(extras["one_step_kernel"]["kernel_us"]
                                                                     / (kernel_ms * 1e3), 3)}
@@ -508,7 +467,7 @@ def main():
         m1 = ref.sums_f64()[0]
         ref.close()
         extras["f64"] = {"GLUPS": round(cells * args.steps / w64 / 1e9, 3),
-                         "hbm_frac": hbm_frac(step_bytes_per_cell("f64", n, k64), cells, ms64 / args.steps),
+                         "hbm_frac": hbm_frac(step_bytes_per_cell("f64", k64), cells, ms64 / args.steps),
                          "steps_per_launch": k64,
                          "mass_drift_rel": abs(m1 - m0) / m0}
         amp = W.taylor_green_decay(n, args.tau, args.steps)
@@ -530,7 +489,7 @@ def main():
             l2.close()
             key = st if st in ("f32", "f32dev") else f"{st}_{rnd}"
             extras[key] = {"GLUPS": round(cells * args.steps / w2 / 1e9, 3),
-                          "hbm_frac": hbm_frac(step_bytes_per_cell(st, n, k2, rnd), cells, ms2 / args.steps),
+                          "hbm_frac": hbm_frac(step_bytes_per_cell(st, k2), cells, ms2 / args.steps),
                           "steps_per_launch": k2,
                           "u_rel_L2_vs_f64": float(np.sqrt(((x - x64) ** 2 + (y - y64) ** 2).sum()) / den),
                           "rho_dev_rel_L2_vs_f64": float(np.sqrt(((r - r64) ** 2).sum()) / rden),
@@ -544,7 +503,7 @@ def main():
         wt, mst = time_steps(lt, args.steps)
         lt.close()
         extras["trt_f32"] = {"GLUPS": round(cells * args.steps / wt / 1e9, 3),
-                             "hbm_frac": hbm_frac(step_bytes_per_cell("f32", n, kt), cells, mst / args.steps),
+                             "hbm_frac": hbm_frac(step_bytes_per_cell("f32", kt), cells, mst / args.steps),
                              "steps_per_launch": kt,
                              "kernel_us": round(mst / args.steps * 1e3, 2), "tau_plus": tp, "tau_minus": tm}
         log(f"[bench] trt: {extras['trt_f32']}")
@@ -557,7 +516,7 @@ def main():
             wo, mso = time_steps(lo, args.steps)
             lo.close()
             extras[key] = {"GLUPS": round(cells * args.steps / wo / 1e9, 3),
-                           "hbm_frac": hbm_frac(step_bytes_per_cell("f32", n, ko), cells, mso / args.steps),
+                           "hbm_frac": hbm_frac(step_bytes_per_cell("f32", ko), cells, mso / args.steps),
                            "steps_per_launch": ko,
                            "kernel_us": round(mso / args.steps * 1e3, 2)}
             log(f"[bench] {key}: {extras[key]}")
@@ -618,7 +577,7 @@ def main():
         cpu["host"] = host_cpu()
         log(f"[bench] cpu baseline {cg:.4f} GLUPS on {threads} threads ({csteps} steps)")
 
-    traffic = load_profile_traffic(f"k_step_tb_{storage}_periodic_fluid_{n}" if temporal
+    traffic = load_profile_traffic(f"k_step_ts_{storage}_periodic_fluid_{n}" if temporal
                                    else f"k_step_{storage}_periodic_fluid_{n}")
     line = {
         "metric": METRIC,
