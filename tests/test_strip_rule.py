@@ -175,3 +175,17 @@ def test_16bit_takes_strips_where_they_are_faster(rule, storage, stochastic, geo
 ])
 def test_remainder_takes_the_faster_of_both(rule, geometry, w, h, strips):
     assert rule("f32", geometry, w, h) == [1, strips]
+
+
+@pytest.mark.parametrize("storage,stochastic,geometry,w,h", [
+    *[("f32", False, g, 2003, 2300) for g in ("periodic", "mask", "mask, zero edge", "porous", "cavity")],
+    *[("f32", False, g, 101, 30011) for g in ("mask, zero edge", "cavity")],
+    *[("f32", False, g, 24641, 163) for g in ("mask, zero edge", "cavity")],
+    ("f32", False, "cavity", 2001, 1499), ("f32", False, "channel", 4100, 3001), ("f32", False, "channel", 3001, 1802),
+    *[(s, r, g, 3001, 3003) for s in ("bf16", "f16") for r in (False, True) for g in ("periodic", "mask", "cavity")],
+    *[(s, r, "channel", 101, 30011) for s in ("bf16", "f16") for r in (False, True)],
+    ("f64", False, "cavity", 1100, 1001), ("f64", False, "channel", 2100, 512),
+])
+def test_lattices_of_the_streaming_tests_take_strips(rule, storage, stochastic, geometry, w, h):
+    """The GPU tests compare the streaming kernel only where a lattice takes it."""
+    assert rule(storage, geometry, w, h, stochastic)[0] == 1
