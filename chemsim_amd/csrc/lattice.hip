@@ -903,11 +903,9 @@ extern "C" int cs_lattice_set_flags(cs_lattice* l, const uint8_t* flags)
             return;
         }
         const int64_t cells = (int64_t)l->w * l->h;
-        bool io = false;
-        for (int64_t d = 0; d < cells; ++d) {
-            CS_REQUIRE(flags[d] <= CS_OUTLET, CS_ERR_ARG, "flag value out of range");
-            io = io || flags[d] >= CS_INLET;
-        }
+        uint8_t top = 0;
+        for (int64_t d = 0; d < cells; ++d) top = std::max(top, flags[d]);
+        CS_REQUIRE(top <= CS_OUTLET, CS_ERR_ARG, "flag value out of range");
         if (!l->flags) {
             const size_t cells = (size_t)l->cpitch * l->h;
             CS_HIP(hipMalloc(&l->flags, cells));
@@ -922,7 +920,7 @@ extern "C" int cs_lattice_set_flags(cs_lattice* l, const uint8_t* flags)
         CS_HIP(hipGetLastError());
         CS_HIP(hipStreamSynchronize(l->stream));
         l->has_flags = true;
-        l->has_io = io;
+        l->has_io = top >= CS_INLET;
     });
 }
 

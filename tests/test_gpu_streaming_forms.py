@@ -109,3 +109,24 @@ def test_channel_with_a_lid(ctx, storage, shape):
     flags[-1, 1:-1] = W.LID
     p = Params(tau=0.62, boundary=capi.CS_BB_HALFWAY, inlet_uy=0.05, outlet_rho=1.0, lid_uy=0.04)
     compare(ctx, w, h, storage, p, flags, 21)
+
+
+@pytest.mark.parametrize("value", [5, 128, 255])
+@pytest.mark.parametrize("at", [0, -1, 1234])
+def test_flags_out_of_range_are_refused(ctx, value, at):
+    """Any cell, any value above CS_OUTLET; the lattice keeps the flags it had."""
+    w, h = 61, 47
+    good = ends(w, h)
+    bad = good.copy()
+    bad.ravel()[at] = value
+    p = Params(tau=0.7, boundary=capi.CS_BB_HALFWAY, lid_uy=0.03)
+    out = []
+    for again in (False, True):
+        with Lattice(ctx, w, h, "f32", p, good) as lat:
+            lat.init_equilibrium(*W.rest_state(w, h))
+            if again:
+                with pytest.raises(capi.ChemsimError, match="flag value out of range"):
+                    lat.set_flags(bad)
+            lat.step(9)
+            out.append(lat.download())
+    np.testing.assert_array_equal(out[0], out[1])
