@@ -22,17 +22,21 @@
 // 463), and 1.3 more with such a last strip (1800 x 1700 235 / 175, 3361 x 3100
 // 563 / 540).  More waves than the device holds take a second, nearly empty round:
 // 229500 x 48 is 2050 strips on 2048 slots, 455 / 366.
-// FP32 Taylor-Green, GLUPS, streaming / regions in registers: 1024^2 110 / 174,
-// 1536^2 187 / 218, 2048^2 198 / 194, 3072^2 263 / 228, 4096^2 306 / 242, 8192^2
-// 350 / 254; half-way cavity, streaming / regions in LDS: 1536^2 118 / 122,
-// 2001 x 1499 139 / 132, 2048^2 160 / 141, 4096^2 243 / 161, 8192^2 288 / 166.
+// us per 8 steps (calls of 8 steps in a row), strips / regions: Taylor-Green 2003 x
+// 2300 148 / 161, 3000^2 250 / 309, 4096^2 417 / 546; half-way cavity 2048^2 183 /
+// 227, 3000^2 308 / 464, 4096^2 517 / 836.  Smaller Taylor-Green lattices in forced
+// strips, GLUPS: 1024^2 110 / 174, 1536^2 187 / 218.
 //
 // FP64 has no region kernels (a region would not fit), and its one-step kernel
 // is bound by HBM at 144 bytes per cell update: GLUPS, streaming / one-step,
 // 512^2 50 / 35, 1024^2 92 / 39, 2048^2 126 / 40, 4096^2 162 / 43, half-way
-// cavity 2048^2 101 / 38.  Lattices of 2^20 cells on take it; below that
-// cs_lattice_temporal_steps goes on reporting one step per launch.  KBC keeps
-// the one-step kernel: its 19 divisions per cell already take as long as the
+// cavity 2048^2 101 / 38.  Lattices of 2^20 cells on take it, of any shape: us per
+// 8 steps 1 x 2^20 1948 / 5320, 4 x 300001 586 / 2731, 49 x 30000 161 / 374 (cavity
+// 286 / 453), 65601 x 17 102 / 291, 98400 x 16 (one wave over the device's) 143 /
+// 376: the one-step kernels compute 64 columns of a narrow lattice too.  The times
+// cross lower (512^2 above); the line stays at the size up to which lattices
+// are replayed from graphs and cs_lattice_temporal_steps reports one step.  KBC
+// keeps the one-step kernel: its 19 divisions per cell already take as long as the
 // memory, and the strips' recomputation would add to them.
 //
 // 16-bit storage rounds every level to 16 bits.  Against the one-step kernel

@@ -18,8 +18,8 @@
 // (level s starts 2 (s - 1) iterations after level 1).  The region variants
 // (lbm_tb.hpp) recompute the halo on all four sides.
 //
-// Bound by VALU issue.  4096^2 FP32 Taylor-Green: 51.2 us per step against
-// 66.9 for the register regions (k_step_tbr), 153 against 201 VALU
+// Bound by VALU issue.  4096^2 FP32 Taylor-Green, 800 steps in a row: 51.8 us per
+// step against 68.2 for the register regions (k_step_tbr), 153 against 201 VALU
 // instructions per kept cell and step, 0.34 against 0.32 of them per SIMD and
 // cycle at two waves per SIMD.  With DPP shifts and v_rcp_f32 instead of the
 // LDS crossbar and recip_newton it ran at 0.27 per cycle, 63 us per step; with

@@ -398,13 +398,15 @@ int cs_set_cells_per_thread(int cells_per_thread);
  * tests and tuning.  No reference counterpart. */
 int cs_set_step_graphs(int enable);
 /* Steps per launch of the temporally blocked step kernels: CS_TEMPORAL_AUTO
- * (the default: 8 steps for every FP32 and FP32-deviation lattice except
- * with the KBC operator -- on 32 x 32 regions for lattices of at most 1024
- * of them, about 512^2, on 64 x 64 regions above, in strips that stream
- * through all 8 levels where those recompute less, about 2048^2 and up; for
- * FP64 lattices of 2^20 cells on (BGK, TRT, Regularized) and large 16-bit
- * lattices in such strips too), 4 or 8 (every FP32 and FP32-deviation
- * lattice, on 64 x 64 regions), or 0 for one step per launch.
+ * (the default: 8 steps for every FP32 and FP32-deviation lattice whose
+ * population buffer is below 4 GiB, about 10900^2, except with the KBC
+ * operator -- on 32 x 32 regions for lattices of at most 1024 of them, about
+ * 512^2, on 64 x 64 regions above, and in strips that stream through all 8
+ * levels where a rule on size and boundary mode finds those faster, about
+ * 2048^2 and up; for FP64 lattices of 2^20 cells on (BGK, TRT, Regularized)
+ * and large 16-bit lattices in such strips too, of any buffer size), 4 or 8
+ * (every FP32 and FP32-deviation lattice below 4 GiB, on 64 x 64 regions), or
+ * 0 for one step per launch.
  * Results are identical either way.  A launch-shape override of
  * cs_set_cells_per_thread selects the one-step kernels instead.
  * Process-wide; for tests and tuning.  No reference counterpart. */
