@@ -10,6 +10,7 @@
 #include <exception>
 #include <memory>
 #include <mutex>
+#include <vector>
 #include <string>
 
 #include "../../include/chemsim.h"
@@ -117,59 +118,107 @@ inline bool is_solid_flag(int t) { return t == CS_WALL || t == CS_LID; }
 
 size_t storage_bytes(int storage);
 
-// Device staging of the moment calls' result planes: one buffer of up to
-// STAGING_KEEP bytes kept from call to call (hipMalloc and hipFree of a 2 MB
-// buffer take about as long as copying it to the host), shared by the handles
-// of a context and freed with the last of them -- one per handle would hold 12
-// to 24 bytes per cell of every lattice that was ever read.
-// A call that finds it taken by another thread's, or needs more, allocates its
-// own for the call.
+// Device staging of the moment calls' result planes, kept from call to call
+// (hipMalloc and hipFree of a 2 MB buffer take about as long as copying it to the
+// host, and hipFree waits for the whole device): as many buffers as calls run at
+// once, of at most STAGING_KEEP bytes together, shared by the handles of a
+// context and freed with the last of them -- one buffer per handle would hold 12
+// to 24 bytes per cell of every lattice that was ever read.  What does not fit is
+// allocated for the call.  Eight threads that each read the velocity of their own
+// 512^2 lattice: 400 us per call of all of them, 905 with one buffer for the
+// context, 1075 with an allocation per call.
 constexpr size_t STAGING_KEEP = (size_t)64 << 20;
-struct KeptStaging {
-    std::mutex mu;  // held by the call that uses the buffer
-    void* p = nullptr;
-    size_t bytes = 0;
-    KeptStaging() = default;
+class KeptStaging {
+public:
+    struct Buf {
+        void* p = nullptr;
+        size_t bytes = 0;
+    };
+    KeptStaging() { idle_.reserve(MOST); }
     KeptStaging(const KeptStaging&) = delete;
     KeptStaging& operator=(const KeptStaging&) = delete;
     ~KeptStaging()
     {
-        if (p) (void)hipFree(p);
+        for (const Buf& b : idle_) (void)hipFree(b.p);
     }
+    // A buffer of at least `bytes` for the caller alone; null if none may be kept for it.
+    Buf take(size_t bytes)
+    {
+        std::vector<Buf> drop;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            auto fit = idle_.end(), big = idle_.end();
+            for (auto i = idle_.begin(); i != idle_.end(); ++i) {
+                if (i->bytes >= bytes && (fit == idle_.end() || i->bytes < fit->bytes)) fit = i;
+                if (big == idle_.end() || i->bytes > big->bytes) big = i;
+            }
+            if (fit != idle_.end()) {
+                const Buf b = *fit;
+                idle_.erase(fit);
+                return b;
+            }
+            if (bytes > STAGING_KEEP) return Buf{};
+            // grow the largest idle one, and drop others while the rest is too much
+            while (big != idle_.end()) {
+                drop.push_back(*big);
+                kept_ -= big->bytes;
+                --count_;
+                idle_.erase(big);
+                big = kept_ + bytes > STAGING_KEEP ? idle_.begin() : idle_.end();
+            }
+            if (kept_ + bytes > STAGING_KEEP || count_ == MOST) bytes = 0;
+            else {
+                kept_ += bytes;
+                ++count_;
+            }
+        }
+        for (const Buf& b : drop) (void)hipFree(b.p);
+        Buf b;
+        if (bytes == 0) return b;
+        const hipError_t e = hipMalloc(&b.p, bytes);
+        if (e != hipSuccess) {
+            std::lock_guard<std::mutex> lk(mu_);
+            kept_ -= bytes;
+            --count_;
+            CS_HIP(e);
+        }
+        b.bytes = bytes;
+        return b;
+    }
+    void give(const Buf& b)
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        idle_.push_back(b);  // within the reserve: count_ <= MOST
+    }
+
+private:
+    static constexpr int MOST = 64;
+    std::mutex mu_;
+    std::vector<Buf> idle_;
+    size_t kept_ = 0;  // bytes of the idle buffers and of those in use
+    int count_ = 0;    // their number
 };
 class Staging {
 public:
     // For work on `stream`, which is waited for before the buffer is given back.
-    Staging(KeptStaging& kept, size_t bytes, hipStream_t stream) : stream_(stream)
+    Staging(KeptStaging& kept, size_t bytes, hipStream_t stream) : kept_(kept), stream_(stream), buf_(kept.take(bytes))
     {
-        if (bytes <= STAGING_KEEP) lock_ = std::unique_lock<std::mutex>(kept.mu, std::try_to_lock);
-        if (!lock_.owns_lock()) {
-            CS_HIP(hipMalloc(&own_, bytes));
-            p_ = own_;
-            return;
-        }
-        if (bytes > kept.bytes) {
-            if (kept.p) (void)hipFree(kept.p);
-            kept.p = nullptr;
-            kept.bytes = 0;
-            CS_HIP(hipMalloc(&kept.p, bytes));
-            kept.bytes = bytes;
-        }
-        p_ = kept.p;
+        if (!buf_.p) CS_HIP(hipMalloc(&own_, bytes));
     }
     ~Staging()
     {
         if (std::uncaught_exceptions() > 0) (void)hipStreamSynchronize(stream_);  // else its user has waited
         if (own_) (void)hipFree(own_);
+        if (buf_.p) kept_.give(buf_);
     }
     Staging(const Staging&) = delete;
     Staging& operator=(const Staging&) = delete;
-    void* get() const { return p_; }
+    void* get() const { return own_ ? own_ : buf_.p; }
 
 private:
-    std::unique_lock<std::mutex> lock_;
+    KeptStaging& kept_;
     hipStream_t stream_;
-    void* p_ = nullptr;
+    KeptStaging::Buf buf_;
     void* own_ = nullptr;
 };
 

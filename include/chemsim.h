@@ -24,8 +24,8 @@
  *    own HIP stream.  Calls on one handle are not re-entrant; different
  *    handles may be used from different threads.
  *  - Handles own their device memory; *_destroy frees it.  The lattices and
- *    batches of a context share one buffer of at most 64 MiB for the results
- *    of the moment calls, kept until the last of them is destroyed.
+ *    batches of a context share buffers of at most 64 MiB together for the
+ *    results of the moment calls, kept until the last of them is destroyed.
  */
 #ifndef CHEMSIM_H
 #define CHEMSIM_H

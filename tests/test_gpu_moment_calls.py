@@ -65,7 +65,7 @@ def _free_bytes():
     return free.value
 
 
-def test_calls_keep_one_bounded_buffer_per_context(ctx):
+def test_calls_keep_bounded_buffers_per_context(ctx):
     """Reading 40 lattices of 1024 x 512 and a batch keeps at most the 64 MiB
     that one context's handles share (12.6 MB for each would be 500 MB), and
     gives it back with the last handle."""
@@ -97,8 +97,8 @@ def test_calls_keep_one_bounded_buffer_per_context(ctx):
 
 
 def test_moment_calls_from_several_threads(ctx):
-    """Lattices of one context read from several threads at once: the shared
-    buffer serves one call at a time, the others have their own."""
+    """Lattices of one context read from several threads at once, each call from a
+    buffer of its own."""
     n, sides = 6, [64, 200, 333, 128, 512, 257]
     lats, want = [], []
     rng = np.random.default_rng(9)
@@ -127,3 +127,41 @@ def test_moment_calls_from_several_threads(ctx):
     for lat in lats:
         lat.close()
     assert not errors, errors
+
+
+def test_threads_do_not_allocate_per_call(ctx):
+    """Six threads that read their own lattices again and again find their buffers
+    kept: the device's free memory never grows meanwhile (with one kept buffer for
+    all, the other five allocated and freed theirs in every call)."""
+    n, side = 6, 512
+    other = Context(0)
+    lats = [Lattice(other, side, side, "f32", Params(tau=0.8)) for _ in range(n)]
+    rest = W.rest_state(side, side)
+    for lat in lats:
+        lat.init_equilibrium(*rest)
+        lat.velocity()
+    start, stop = threading.Barrier(n), threading.Event()
+    seen = [_free_bytes()]
+
+    def read(k):
+        start.wait()
+        for _ in range(200):
+            lats[k].velocity()
+
+    def watch():
+        while not stop.is_set():
+            seen.append(_free_bytes())
+
+    watcher = threading.Thread(target=watch)
+    watcher.start()
+    threads = [threading.Thread(target=read, args=(k,)) for k in range(n)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    stop.set()
+    watcher.join()
+    for lat in lats:
+        lat.close()
+    assert len(seen) > 20
+    assert all(b <= a for a, b in zip(seen, seen[1:])), sorted(set(seen))
