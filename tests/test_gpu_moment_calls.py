@@ -1,5 +1,6 @@
 """The moment calls' way to the host: a small lattice's planes cross in one
 copy, and what a call keeps on the device is bounded."""
+import gc
 import threading
 import time
 
@@ -79,6 +80,7 @@ def test_calls_keep_bounded_buffers_per_context(ctx):
     for i in range(3):
         batch.init_equilibrium(i, *rest)
     lats[0].sync()
+    gc.collect()
     before = _free_bytes()
     for lat in lats:
         lat.moments_f64()
@@ -140,6 +142,7 @@ def test_threads_do_not_allocate_per_call(ctx):
     for lat in lats:
         lat.init_equilibrium(*rest)
         lat.velocity()
+    gc.collect()  # handles that earlier tests dropped free their memory now
     start, stop = threading.Barrier(n), threading.Event()
     seen = [_free_bytes()]
 

@@ -130,3 +130,28 @@ def test_flags_out_of_range_are_refused(ctx, value, at):
             lat.step(9)
             out.append(lat.download())
     np.testing.assert_array_equal(out[0], out[1])
+
+
+def test_buffers_above_4_gib(ctx):
+    """FP64 strips address rows from 64-bit bases: a population buffer of 4.4e9
+    bytes, eight steps in one launch and four in another against twelve one-step
+    launches, every cell's density and velocity."""
+    w, h = 7800, 7800
+    y, x = np.arange(h)[:, None], np.arange(w)[None, :]
+    rho = 1 + 0.01 * np.sin(0.013 * y + 0.011 * x)
+    ux, uy = 0.03 * np.cos(0.017 * y) * np.sin(0.012 * x), 0.03 * np.sin(0.009 * y) * np.cos(0.014 * x)
+    flags = np.zeros((h, w), np.uint8)
+    flags[-2:, ::97] = W.WALL
+    out = []
+    try:
+        for k in (capi.CS_TEMPORAL_AUTO, 0):
+            capi.call("cs_set_temporal_steps", k)
+            with Lattice(ctx, w, h, "f64", Params(tau=0.7, edge=capi.CS_EDGE_PERIODIC), flags) as lat:
+                assert lat.temporal_steps() == (8 if k else 1)
+                lat.init_equilibrium(rho, ux, uy)
+                lat.step(12)
+                out.append(lat.moments_f64())
+    finally:
+        capi.call("cs_set_temporal_steps", capi.CS_TEMPORAL_AUTO)
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
