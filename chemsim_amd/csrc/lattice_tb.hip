@@ -177,11 +177,3 @@ extern "C" int cs_set_temporal_steps(int k)
         g_tb_steps.store(k, std::memory_order_relaxed);
     });
 }
-
-// The library's Makefile compiles the streaming kernel's units on their own,
-// in parallel; a build that lists only this one gets them here.
-#ifndef CS_TS_UNITS
-#include "lattice_ts.hip"
-#include "lattice_ts_f64.hip"
-#include "lattice_ts_16.hip"
-#endif

@@ -1,4 +1,5 @@
-"""The sanitizer build rebuilds when any file it compiles has changed."""
+"""The sanitizer build compiles the library's units and rebuilds when any file it
+compiles has changed."""
 import os
 import re
 import subprocess
@@ -28,3 +29,10 @@ def test_sanitizer_build_follows_every_included_file(tmp_path):
     for unit in units:
         missing = _included(os.path.join(CSRC, unit), set()) - listed
         assert not missing, (unit, sorted(os.path.relpath(f, CSRC) for f in missing))
+
+
+def test_sanitizer_build_has_the_librarys_units():
+    def sources(path, name):
+        return set(re.search(rf"^{name} := (.*)$", open(path).read(), re.M).group(1).split())
+    lib = sources(os.path.join(CSRC, "Makefile"), "LBM_SRCS") | {"cnn.hip"}
+    assert sources(os.path.join(HERE, "cpu_hip", "Makefile"), "LIB_SRCS") == lib
