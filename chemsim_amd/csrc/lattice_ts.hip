@@ -55,7 +55,8 @@
 //   x 96 bf16 to nearest 1350 / 1274; f16 to nearest is faster all the same, 975 /
 //   1262;
 //   inlets and outlets with stochastic rounding (f16 / bf16 2048^2 364 / 331, 379 /
-//   331; 3000^2 634 / 628, 659 / 627; 4096^2 1073 / 1131, 1121 / 1126);
+//   331; 3000^2 634 / 628, 659 / 627; 4096^2 1073 / 1131, 1121 / 1126; bf16 3710 x
+//   3135 819 / 780);
 //   a solid mask: bf16 stochastic 2048^2 with a few obstacles 294 / 271, with 2%
 //   of random cells 306 / 272, 3000^2 520 / 536; bf16 to nearest 1500^2 182 / 170,
 //   1800 x 1700 220 / 223; f16 stochastic 4100 x 1517 396 / 382, 9100 x 817 466 / 468;

@@ -112,7 +112,7 @@ inline bool ts_takes_16(const StripCase& c)
     const double cost = stream * (1 + (bf16 || c.half ? 1.5 : 1.0) * std::max(0.0, idle - 1.05)) *
                         (ts_two_wall_strips(c) ? 1.3 : 1.0);
     const double tiles = (double)((c.w + 255) / 256 * 256) / c.w;
-    if (c.io && sr) return cost / tiles < 1.31;
+    if (c.io && sr) return cost / tiles < (bf16 ? 1.24 : 1.31);
     if (c.half) return cost < (sr ? most : 2.0);
     if (c.mask) return cost / tiles < (!sr ? 1.75 : bf16 ? 1.375 : 1.4);
     return cost < most;

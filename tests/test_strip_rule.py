@@ -113,6 +113,8 @@ def test_fp32_takes_strips_where_they_are_faster(rule, storage, geometry, w, h):
     ("f16", True, "channel", 2048, 2048),    # 330 / 363
     ("bf16", True, "channel", 2048, 2048),   # 329 / 379
     ("bf16", True, "channel", 3000, 3000),   # 627 / 659
+    ("bf16", True, "channel", 2671, 3271),   # 608 / 645
+    ("bf16", True, "channel", 3710, 3135),   # 780 / 819
     ("bf16", True, "cavity", 2353, 3000),    # 539 / 577, one column in the last strip
     ("f16", True, "cavity", 2353, 3000),     # 540 / 555
     ("bf16", True, "cavity", 3361, 3100),    # 737 / 779
